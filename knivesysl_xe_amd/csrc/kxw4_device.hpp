@@ -21,10 +21,19 @@
 
 namespace kxw4 {
 
+// Kernels that keep direct global->LDS loads in flight read LDS through these
+// vector types and plain scalars, never through HIP's own float4 / uint2: for
+// a read of those class types the compiler assumes that it may depend on the
+// loads in flight and waits for all of them (s_waitcnt vmcnt(0)), which made
+// every step of the reference-mode and W4A4 GEMMs wait for the stage it had
+// just requested (reference mode T = 65-192, N = 5120, K = 17408: 166 ->
+// 147 us; T = 512: 277 -> 257 us; W4A4 T = 512: 165 -> 159 us).
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int kTileK = 128;        // K extent of one packed weight tile
 constexpr int kTileBytes = 1024;   // 16 rows x 128 K x 4 bits

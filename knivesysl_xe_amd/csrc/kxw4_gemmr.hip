@@ -303,7 +303,7 @@ __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemmr_kernel(const GemmArgs 
         auto read_ws = [&](int g, uint32_t (&w)[8]) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const uint2 v = *reinterpret_cast<const uint2 *>(sb + ws_lds + (q >> 1) * GPS * 32 + (q & 1) * 16 + g * 32);
+                const v2u v = *reinterpret_cast<const v2u *>(sb + ws_lds + (q >> 1) * GPS * 32 + (q & 1) * 16 + g * 32);
                 w[2 * q] = v.x;
                 w[2 * q + 1] = v.y;
             }
@@ -314,8 +314,8 @@ __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemmr_kernel(const GemmArgs 
             const int u = i / NT, j = i % NT, c = u >> 1, h = u & 1;
             const int s0 = ((4 * c + 2 * kg) ^ tsw) * 16 + 8 * h;
             const int s1 = ((4 * c + 2 * kg + 1) ^ tsw) * 16 + 8 * h;
-            const uint2 b0 = *reinterpret_cast<const uint2 *>(sb + a_row + j * 32 * kTileK + s0);
-            const uint2 b1 = *reinterpret_cast<const uint2 *>(sb + a_row + j * 32 * kTileK + s1);
+            const v2u b0 = *reinterpret_cast<const v2u *>(sb + a_row + j * 32 * kTileK + s0);
+            const v2u b1 = *reinterpret_cast<const v2u *>(sb + a_row + j * 32 * kTileK + s1);
             B.x = (int)b0.x;
             B.y = (int)b0.y;
             B.z = (int)b1.x;

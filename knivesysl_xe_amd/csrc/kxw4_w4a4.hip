@@ -256,7 +256,7 @@ __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void w4a4_kernel(const W4a4Args a
             for (int u = 0; u < UPS; ++u)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const float4 v = *reinterpret_cast<const float4 *>(sb + asoff_lds + (u * BM + 32 * ib + 8 * q) * 4);
+                    const v4f v = *reinterpret_cast<const v4f *>(sb + asoff_lds + (u * BM + 32 * ib + 8 * q) * 4);
                     asv[u][4 * q] = v.x;
                     asv[u][4 * q + 1] = v.y;
                     asv[u][4 * q + 2] = v.z;
