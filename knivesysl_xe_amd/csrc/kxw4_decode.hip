@@ -1,6 +1,8 @@
-// kxw4_decode.hip — decode-shaped projections (T <= 64 tokens): the GEMV
-// (kernels_dpas.cpp:586-675), the fan-out GEMV (945-1102) and the batched /
-// packed GEMM at small T (1334-1490).
+// kxw4_decode.hip — dispatch of the decode-shaped projections (T <= 64
+// tokens) and the K-parallel kernel: the GEMV (kernels_dpas.cpp:586-675), the
+// fan-out GEMV (945-1102) and the batched / packed GEMM at small T
+// (1334-1490) in the modes the strip kernel (kxw4_strip.hip) is not built
+// for, and the debug partials.
 //
 // The integer work and the float chain are decoupled:
 //   * a work-group owns one 16-row row-group (and a slice of at most `ts`
@@ -350,28 +352,39 @@ int device_cus() {
 }
 
 int launch_decode(DecodeArgs &a, bool debug, hipStream_t st) {
-    // Up to 16 tokens go to the row-wave kernel, the rest stay here. The
-    // decode_kernel option forces the K-parallel kernel (kparallel) or
-    // prefers the row-wave kernel (rowwave); the tests use both to cover
-    // every kernel at the decode shapes.
-    // W8 and K16 weights run on the row-wave kernel only; 1 hands the shape
+    // Every mode the strip kernel takes goes there, but for one: per-token
+    // launches of 3-16 tokens over many rows stay on the row-wave kernel,
+    // which cuts the rows evenly over the CUs and stages the activations
+    // once per work-group (8 tokens, K = 5120, 34,816 rows: 18.5 against
+    // 20.9 us; 17,408 rows: 12.4 against 11.3 us). The decode_kernel option
+    // forces the K-parallel kernel below (kparallel) or prefers the row-wave
+    // kernel (rowwave, as a rowwave_* option does); the modes the strip
+    // kernel is not built for (per-token activations with zero points or
+    // group 32, K32 blocks with plain FP16 scales) run on those two.
+    const int force = options().decode_kernel;
+    const bool rw_opt = options().rowwave_spw || options().rowwave_ring || options().rowwave_k;
+    if (!debug && force == kDecodeAuto && !rw_opt && strip_takes(a.group, a.block, a.scale_enc, a.T, a.K)) {
+        int rgs = 0;
+        for (int i = 0; i < a.count; ++i) rgs += a.w[i].M / 16;
+        if (a.block == 0 && a.T > 2 && a.T <= 16 && rgs > 6 * device_cus()) {
+            const int r = launch_rowwave(a, st);
+            if (r != 1) return r;
+        }
+        return launch_strip_classes(a, st);
+    }
+    // W8 and K16 weights have no K-parallel instance; 1 hands the shape
     // back to the caller (the GEMM path for W8)
     if (a.w8 || a.group == 16) return debug ? 1 : launch_rowwave(a, st);
-    const int force = options().decode_kernel;
     bool no_rowwave = force == kDecodeKParallel;
-    // Per-token weights with at most 8 tokens and no more row-groups than
-    // CUs stay here: one work-group per row-group whose waves read
-    // consecutive kilobytes beats the row-wave kernel's per-split streams
-    // when every CU holds at most one row-group (T = 4: 5.5 against 6.4 us
-    // at M = K = 4096) -- except for one or two tokens with at most 8 splits
-    // of at most 8 tiles each, where the row-wave kernel's short chains and
-    // single ring win (cfg0: 5.3 against 5.4 us; K = 2048: 4.6 against 5.0).
-    if (force != kDecodeRowwave && a.block == 0 && a.scale_enc == 0 && a.T <= 8) {
+    if (force == kDecodeAuto && a.block == 0 && a.scale_enc == 0 && a.T <= 8) {
+        // per-token group 32 with at most one row-group per CU: one
+        // work-group per row-group whose waves read consecutive kilobytes
+        // beats the row-wave kernel's per-split streams, except for one or
+        // two tokens with at most 8 splits of at most 8 tiles each
         int rgs = 0;
         for (int i = 0; i < a.count; ++i) rgs += a.w[i].M / 16;
         const int S = a.w[0].seg_split[0];
-        const bool short_rowwave = a.T <= 2 && S <= 8 && (a.K / kTileK) <= 8 * S;
-        if (rgs <= device_cus() && !short_rowwave) no_rowwave = true;
+        no_rowwave = rgs <= device_cus() && !(a.T <= 2 && S <= 8 && (a.K / kTileK) <= 8 * S);
     }
     if (!debug && !no_rowwave) {
         const int r = launch_rowwave(a, st);

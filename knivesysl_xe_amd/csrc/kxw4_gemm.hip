@@ -417,15 +417,89 @@ static void launch_w8(const GemmArgs &a, bool splits, bool debug, dim3 grid, hip
     else hipLaunchKernelGGL((gemm_kernel<2, 32, 1, false, false, true>), grid, block, 0, st, a);
 }
 
-int launch_gemm(GemmArgs &a, bool debug, hipStream_t st) {
-    // The one-split modes go to the large-tile kernels (per-token: gemm3;
-    // K32 activation blocks: gemmr); the gemm_kernel option keeps them here
-    // (the tests cover both).
-    if (!debug && options().gemm_kernel != kGemmGeneral && !a.w8) {
+// The segments [s0, s1) of a projection whose weights in `mask` are planned
+// with one split, as a projection of its own (outputs depend on their own
+// token row only).
+static GemmArgs sub_gemm(const GemmArgs &a, unsigned mask, int s0, int s1) {
+    GemmArgs g = a;
+    const int t0 = s0 ? a.seg_end[s0 - 1] : 0;
+    g.T = a.seg_end[s1 - 1] - t0;
+    g.count = 0;
+    for (int i = 0; i < a.count; ++i) {
+        if (!(mask >> i & 1)) continue;
+        GemmWeight &w = g.w[g.count++];
+        w = a.w[i];
+        w.y = static_cast<uint8_t *>(a.w[i].y) + (size_t)t0 * a.w[i].M * (a.y_bf16 ? 2 : 4);
+        w.seg_split[0] = 1;
+    }
+    g.seg_count = 1;
+    g.seg_end[0] = g.T;
+    const size_t per = a.block ? (size_t)a.K / a.block : 1;  // activation scales per token
+    g.q = a.q + (size_t)t0 * a.K;
+    g.ascale = a.ascale + (size_t)t0 * per;
+    g.asum = a.asum ? a.asum + (size_t)t0 * (a.K / 32) : nullptr;
+    g.residual = a.residual ? a.residual + (size_t)t0 * a.w[0].M : nullptr;
+    return g;
+}
+
+// One-split projections of up to this many 16-row x 32-token strips run on
+// the strip kernel, whose grid still fills the chip where the large tiles
+// leave CUs idle (per-token N = 5120, K = 17408, T = 256, 2,560 strips: 58
+// against 81 us; N = 17408, K = 5120, T = 128, 4,352 strips: 35 against 35
+// us, T = 256: 53 against 46; block mode N = 17408, T = 256, 8,704 strips:
+// 107 against 120 us). W8 has no large-tile kernel, so all of it goes there.
+static long long strip_limit(const GemmArgs &a) {
+    if (a.w8) return 1ll << 62;
+    return a.block == 32 ? 9000 : 4000;
+}
+
+static int launch_one_split(GemmArgs &a, hipStream_t st) {
+    long long strips = 0;
+    for (int i = 0; i < a.count; ++i) strips += (long long)(a.w[i].M / 16) * ((a.T + 31) / 32);
+    if (strips > strip_limit(a)) {
         int r = launch_gemm3(a, st);
-        if (r != 1) return r;
-        r = launch_gemmr(a, st);
-        if (r != 1) return r;
+        if (r == 1) r = launch_gemmr(a, st);
+        if (r != 1) return r;                                // (1: past the large tiles' 32-bit offsets)
+    }
+    StripArgs s = strip_args(a, kVarGemm, 1);
+    return launch_strip(s, st);
+}
+
+int launch_gemm(GemmArgs &a, bool debug, hipStream_t st) {
+    // Every split count runs on the strip kernel; what is planned with one
+    // split goes to the large tiles where it fills them (per-token: gemm3;
+    // K32 activation blocks: gemmr). The gemm_kernel option keeps everything
+    // here (the tests cover both), a gemm3_tile / gemmr_tile option asks for
+    // the large tiles.
+    if (!debug && options().gemm_kernel != kGemmGeneral) {
+        const bool tile = a.block == 0 ? options().gemm3_tile >= 0 : options().gemmr_tile >= 0;
+        if (tile || !strip_takes(a.group, a.block, a.scale_enc, a.T, a.K)) {
+            int r = launch_gemm3(a, st);
+            if (r != 1) return r;
+            r = launch_gemmr(a, st);
+            if (r != 1) return r;
+        } else {
+            for (int S = 16; S > 1; S >>= 1) {
+                StripArgs s = strip_args(a, kVarGemm, S);
+                const int r = s.entries ? launch_strip(s, st) : 0;
+                if (r) return r;
+            }
+            // runs of neighbouring segments whose one-split weights are the same
+            auto ones = [&](int s) {
+                unsigned m = 0;
+                for (int i = 0; i < a.count; ++i) m |= (unsigned)(a.w[i].seg_split[s] == 1) << i;
+                return m;
+            };
+            for (int s0 = 0, s1; s0 < a.seg_count; s0 = s1) {
+                const unsigned m = ones(s0);
+                for (s1 = s0 + 1; s1 < a.seg_count && ones(s1) == m; ++s1) {}
+                if (!m) continue;
+                GemmArgs g = sub_gemm(a, m, s0, s1);
+                const int r = launch_one_split(g, st);
+                if (r) return r;
+            }
+            return 0;
+        }
     }
     bool splits = false;
     int nt = 0;

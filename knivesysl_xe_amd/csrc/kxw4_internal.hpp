@@ -112,6 +112,61 @@ int launch_decode(DecodeArgs &a, bool debug, hipStream_t st);
 // Return 1 (nothing launched) when the shape is outside the kernel's range.
 int launch_rowwave(DecodeArgs &a, hipStream_t st);
 int launch_gemm(GemmArgs &a, bool debug, hipStream_t st);
+
+struct StripWeight {
+    const uint8_t *codes;
+    const uint16_t *scales;
+    void *y;
+    int M;
+};
+// tokens [t0, t1) of weight w; blk: its first work-group (set by the launcher)
+struct StripEntry {
+    int w, t0, t1, blk;
+};
+struct StripArgs {
+    StripWeight w[kMaxWeights];
+    const int8_t *q;
+    const float *ascale;
+    const float *residual;
+    int K, group, block, scale_enc, y_bf16, variant;
+    int S;                            // split count of every entry
+    int SW;                           // streams per work-group (set by the launcher)
+    int entries;
+    StripEntry e[kMaxWeights * kMaxSegments];
+};
+// the modes the strip kernel is built for
+bool strip_takes(int group, int block, int scale_enc, long long T, int K);
+int launch_strip(StripArgs &a, hipStream_t st);
+// one launch per split count of the projection
+int launch_strip_classes(const DecodeArgs &a, hipStream_t st);
+
+// The (weight, segment) pairs of a projection whose split count is S, as
+// entries (neighbouring segments of one weight merge); A: DecodeArgs or
+// GemmArgs.
+template <class A>
+StripArgs strip_args(const A &a, int variant, int S) {
+    StripArgs s{};
+    for (int i = 0; i < a.count; ++i) {
+        s.w[i] = StripWeight{a.w[i].codes, a.w[i].scales, a.w[i].y, a.w[i].M};
+        for (int g = 0; g < a.seg_count; ++g) {
+            if (a.w[i].seg_split[g] != S) continue;
+            const int t0 = g ? a.seg_end[g - 1] : 0, t1 = a.seg_end[g];
+            if (s.entries && s.e[s.entries - 1].w == i && s.e[s.entries - 1].t1 == t0) s.e[s.entries - 1].t1 = t1;
+            else s.e[s.entries++] = StripEntry{i, t0, t1, 0};
+        }
+    }
+    s.q = a.q;
+    s.ascale = a.ascale;
+    s.residual = a.residual;
+    s.K = a.K;
+    s.group = a.group;
+    s.block = a.block;
+    s.scale_enc = a.scale_enc;
+    s.y_bf16 = a.y_bf16;
+    s.variant = variant;
+    s.S = S;
+    return s;
+}
 // Returns 1 (nothing launched) outside the per-token, one-split-per-token mode.
 int launch_gemm3(GemmArgs &a, hipStream_t st);
 // Returns 1 (nothing launched) outside the reference mode (K32 activation

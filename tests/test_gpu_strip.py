@@ -1,0 +1,114 @@
+"""The strip kernel (csrc/kxw4_strip.hip) at the edges of its tiles, stages
+and split plans, against the oracle: int32 partials and the order of every
+FP32 step are fixed, so the outputs must be the oracle's bits."""
+import numpy as np
+import pytest
+import torch
+
+from knivesysl_xe_amd import ops
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(autouse=True, scope="module")
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    O.set_num_threads(16)
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+
+# group, activation block, scale encoding
+MODES = {"token128": (128, 0, O.SCALE_FP16), "token64": (64, 0, O.SCALE_FP16),
+         "block32": (32, 32, O.SCALE_FP16_ZP4), "block64": (64, 32, O.SCALE_FP16_ZP4), "w8": (32, 32, None),
+         "k16": (16, 32, O.SCALE_FP16_ZP4)}
+
+
+def weight(rng, mode, M, K):
+    group, _, enc = MODES[mode]
+    lim = (-128, 128) if mode == "w8" else (-8, 8)
+    codes = rng.integers(*lim, (M, K)).astype(np.int8)
+    scales = (np.abs(rng.standard_normal((M, K // group))) * 0.02).astype(np.float16).view(np.uint16)
+    if enc == O.SCALE_FP16_ZP4:
+        scales = ((scales & 0xFFF0) | (rng.integers(-8, 8, scales.shape) & 0xF)).astype(np.uint16)
+    bits = dev(scales.view(np.int16))
+    w = ops.W4Weight.from_codes_s8(dev(codes), bits) if mode == "w8" else ops.W4Weight.from_codes(dev(codes), bits, group, enc)
+    return codes, scales, w
+
+
+def oracle(mode, codes, scales, act, variant, splits, **kw):
+    group, block, enc = MODES[mode]
+    return O.project(codes, scales, group, O.SCALE_S8 if mode == "w8" else enc, *act, block, variant, splits, **kw)
+
+
+def check(y, ref, what):
+    bits = np.uint16 if y.dtype == torch.bfloat16 else np.uint32
+    got = (y.view(torch.int16) if y.dtype == torch.bfloat16 else y).cpu().numpy().view(bits)
+    assert np.array_equal(got, ref.view(bits)), f"{what}: {np.count_nonzero(got != ref.view(bits))} of {got.size} differ"
+
+
+# tokens around the tile sizes (1, 2, 8, 16, 32); one K tile, an odd number of
+# tiles (a half-empty last stage) and enough for whole stages; row-groups that
+# do not divide the row waves; splits that end inside a tile (K = 640: 20 K32
+# units in 16 parts) and splits with no unit at all (K = 128 in 16)
+@pytest.mark.parametrize("mode", ["token128", "token64", "block32", "block64", "w8"])
+@pytest.mark.parametrize("T,M,K,forced", [
+    (1, 16, 128, 1), (2, 48, 384, 2), (3, 80, 640, 16), (8, 144, 640, 4), (9, 16, 128, 16), (16, 80, 1152, 8),
+    (17, 48, 384, 1), (31, 80, 640, 2), (33, 144, 1152, 16), (64, 16, 640, 4), (70, 176, 384, 1), (130, 48, 640, 8)])
+def test_strip_gemm_edges(mode, T, M, K, forced):
+    rng = np.random.default_rng(T * M + K)
+    codes, scales, w = weight(rng, mode, M, K)
+    block = MODES[mode][1]
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    res = rng.standard_normal((T, M)).astype(np.float32)
+    a, act = ops.quantize_act(dev(x), block), O.quantize_act(x, block)
+    sp = O.segment_splits(T, M, K, None, forced)
+    check(ops.gemm(w, a, residual=dev(res), forced_splits=forced),
+          oracle(mode, codes, scales, act, O.VAR_GEMM, sp, residual=res), f"{mode} T={T}")
+    check(ops.gemm(w, a, torch.bfloat16, forced_splits=forced),
+          oracle(mode, codes, scales, act, O.VAR_GEMM, sp, out_bf16=True), f"{mode} T={T} bf16")
+
+
+# the GEMV's two accumulators, the K16 halves and the fan-out's association
+@pytest.mark.parametrize("mode,T,M,K,splits", [
+    ("token128", 1, 48, 640, 1), ("token128", 40, 80, 384, 2), ("token64", 2, 80, 1152, 8), ("token64", 33, 48, 640, 16),
+    ("block32", 1, 80, 640, 16), ("block64", 17, 48, 384, 1), ("block32", 64, 16, 1152, 4), ("w8", 1, 48, 384, 2),
+    ("w8", 16, 80, 640, 16), ("k16", 1, 48, 640, 16), ("k16", 2, 80, 384, 1), ("k16", 8, 16, 1152, 8),
+    ("k16", 16, 144, 128, 4)])
+def test_strip_gemv(mode, T, M, K, splits):
+    rng = np.random.default_rng(T * M + K + splits)
+    codes, scales, w = weight(rng, mode, M, K)
+    block = MODES[mode][1]
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    a, act = ops.quantize_act(dev(x), block), O.quantize_act(x, block)
+    check(ops.gemv(w, a, splits=splits), oracle(mode, codes, scales, act, O.VAR_GEMV, splits), f"{mode} gemv")
+    if mode not in ("w8", "k16"):
+        c2, s2, w2 = weight(rng, mode, 32, K)
+        ys = ops.gemv_fanout([w, w2], a)
+        S = O.gemv_splits((M + 32) // 16)
+        for c, s, y in ((codes, scales, ys[0]), (c2, s2, ys[1])):
+            check(y, oracle(mode, c, s, act, O.VAR_FANOUT, S), f"{mode} fan-out")
+
+
+# packed prompts whose segments have different split counts, and weights of a
+# fan-out that are planned apart: strips of several split counts beside the
+# large tiles, over token ranges that start and end anywhere
+@pytest.mark.parametrize("mode", ["token128", "token64", "block32", "w8"])
+@pytest.mark.parametrize("rows,segs", [([4096], [9, 61, 300, 5]), ([8192, 48], [70, 3, 129]), ([1024, 2048], [250, 17, 40])])
+def test_strip_packed_segments(mode, rows, segs):
+    rng = np.random.default_rng(sum(rows) + sum(segs))
+    K, T = 384, sum(segs)
+    off = [0] + [int(o) for o in np.cumsum(segs)]
+    block = MODES[mode][1]
+    ws = [weight(rng, mode, M, K) for M in rows]
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    a, act = ops.quantize_act(dev(x), block), O.quantize_act(x, block)
+    ys = ops.gemm_fanout([w for _, _, w in ws], a, offsets=off)
+    for (c, s, _), y in zip(ws, ys):
+        sp = O.segment_splits(T, c.shape[0], K, off)
+        check(y, oracle(mode, c, s, act, O.VAR_GEMM, sp), f"{mode} rows={c.shape[0]}")
