@@ -370,7 +370,8 @@ int launch_decode(DecodeArgs &a, bool debug, hipStream_t st) {
             const int r = launch_rowwave(a, st);
             if (r != 1) return r;
         }
-        return launch_strip_classes(a, st);
+        StripArgs s = strip_args(a, a.variant, 1, 16);
+        return launch_strip(s, st);
     }
     // W8 and K16 weights have no K-parallel instance; 1 hands the shape
     // back to the caller (the GEMM path for W8)

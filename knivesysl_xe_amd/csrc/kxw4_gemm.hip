@@ -453,16 +453,10 @@ static long long strip_limit(const GemmArgs &a) {
     return a.block == 32 ? 9000 : 4000;
 }
 
-static int launch_one_split(GemmArgs &a, hipStream_t st) {
-    long long strips = 0;
-    for (int i = 0; i < a.count; ++i) strips += (long long)(a.w[i].M / 16) * ((a.T + 31) / 32);
-    if (strips > strip_limit(a)) {
-        int r = launch_gemm3(a, st);
-        if (r == 1) r = launch_gemmr(a, st);
-        if (r != 1) return r;                                // (1: past the large tiles' 32-bit offsets)
-    }
-    StripArgs s = strip_args(a, kVarGemm, 1);
-    return launch_strip(s, st);
+static long long strips_of(const StripArgs &s) {
+    long long n = 0;
+    for (int i = 0; i < s.entries; ++i) n += (long long)(s.w[s.e[i].w].M / 16) * ((s.e[i].t1 - s.e[i].t0 + 31) / 32);
+    return n;
 }
 
 int launch_gemm(GemmArgs &a, bool debug, hipStream_t st) {
@@ -479,11 +473,14 @@ int launch_gemm(GemmArgs &a, bool debug, hipStream_t st) {
             r = launch_gemmr(a, st);
             if (r != 1) return r;
         } else {
-            for (int S = 16; S > 1; S >>= 1) {
-                StripArgs s = strip_args(a, kVarGemm, S);
-                const int r = s.entries ? launch_strip(s, st) : 0;
+            StripArgs split = strip_args(a, kVarGemm, 2, 16);
+            if (split.entries) {
+                const int r = launch_strip(split, st);
                 if (r) return r;
             }
+            StripArgs one = strip_args(a, kVarGemm, 1, 1);
+            if (!one.entries) return 0;
+            if (strips_of(one) <= strip_limit(a)) return launch_strip(one, st);
             // runs of neighbouring segments whose one-split weights are the same
             auto ones = [&](int s) {
                 unsigned m = 0;
@@ -495,7 +492,13 @@ int launch_gemm(GemmArgs &a, bool debug, hipStream_t st) {
                 for (s1 = s0 + 1; s1 < a.seg_count && ones(s1) == m; ++s1) {}
                 if (!m) continue;
                 GemmArgs g = sub_gemm(a, m, s0, s1);
-                const int r = launch_one_split(g, st);
+                StripArgs s = strip_args(g, kVarGemm, 1, 1);
+                int r = 1;
+                if (strips_of(s) > strip_limit(g)) {
+                    r = launch_gemm3(g, st);
+                    if (r == 1) r = launch_gemmr(g, st);
+                }
+                if (r == 1) r = launch_strip(s, st);         // (few strips, or past the large tiles' 32-bit offsets)
                 if (r) return r;
             }
             return 0;

@@ -119,9 +119,10 @@ struct StripWeight {
     void *y;
     int M;
 };
-// tokens [t0, t1) of weight w; blk: its first work-group (set by the launcher)
+// tokens [t0, t1) of weight w, planned with S splits; blk: its first
+// work-group (set by the launcher)
 struct StripEntry {
-    int w, t0, t1, blk;
+    int w, t0, t1, S, blk;
 };
 struct StripArgs {
     StripWeight w[kMaxWeights];
@@ -129,30 +130,31 @@ struct StripArgs {
     const float *ascale;
     const float *residual;
     int K, group, block, scale_enc, y_bf16, variant;
-    int S;                            // split count of every entry
-    int SW;                           // streams per work-group (set by the launcher)
+    int waves, same_s;                // waves per work-group, whether every entry has one S (set by the launcher)
     int entries;
     StripEntry e[kMaxWeights * kMaxSegments];
 };
 // the modes the strip kernel is built for
 bool strip_takes(int group, int block, int scale_enc, long long T, int K);
 int launch_strip(StripArgs &a, hipStream_t st);
-// one launch per split count of the projection
-int launch_strip_classes(const DecodeArgs &a, hipStream_t st);
 
-// The (weight, segment) pairs of a projection whose split count is S, as
-// entries (neighbouring segments of one weight merge); A: DecodeArgs or
-// GemmArgs.
+// The (weight, segment) pairs of a projection whose split count lies in
+// [smin, smax], as entries (neighbouring segments of one weight and split
+// count merge); A: DecodeArgs or GemmArgs.
 template <class A>
-StripArgs strip_args(const A &a, int variant, int S) {
-    StripArgs s{};
+StripArgs strip_args(const A &a, int variant, int smin, int smax) {
+    StripArgs s;
+    s.entries = 0;
+    for (int i = 0; i < kMaxWeights; ++i)
+        s.w[i] = i < a.count ? StripWeight{a.w[i].codes, a.w[i].scales, a.w[i].y, a.w[i].M} : StripWeight{};
     for (int i = 0; i < a.count; ++i) {
-        s.w[i] = StripWeight{a.w[i].codes, a.w[i].scales, a.w[i].y, a.w[i].M};
         for (int g = 0; g < a.seg_count; ++g) {
-            if (a.w[i].seg_split[g] != S) continue;
+            const int S = a.w[i].seg_split[g];
+            if (S < smin || S > smax) continue;
             const int t0 = g ? a.seg_end[g - 1] : 0, t1 = a.seg_end[g];
-            if (s.entries && s.e[s.entries - 1].w == i && s.e[s.entries - 1].t1 == t0) s.e[s.entries - 1].t1 = t1;
-            else s.e[s.entries++] = StripEntry{i, t0, t1, 0};
+            StripEntry *e = s.entries ? &s.e[s.entries - 1] : nullptr;
+            if (e && e->w == i && e->t1 == t0 && e->S == S) e->t1 = t1;
+            else s.e[s.entries++] = StripEntry{i, t0, t1, S, 0};
         }
     }
     s.q = a.q;
@@ -164,7 +166,6 @@ StripArgs strip_args(const A &a, int variant, int S) {
     s.scale_enc = a.scale_enc;
     s.y_bf16 = a.y_bf16;
     s.variant = variant;
-    s.S = S;
     return s;
 }
 // Returns 1 (nothing launched) outside the per-token, one-split-per-token mode.

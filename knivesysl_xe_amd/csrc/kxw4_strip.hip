@@ -70,6 +70,9 @@ struct StShape {
     // dealt to the row waves
     static constexpr int PA = U * 8 * TT, A_LOADS = ((PA + 63) / 64 + RW - 1) / RW;
     static constexpr int PS = U * TT, S_LOADS = ((PS + 63) / 64 + RW - 1) / RW;
+    // loads a wave issues per stage when it issues all of them (RW = 1)
+    static constexpr int LOADS = U * TB + A_LOADS + 1 + (BLK ? S_LOADS : 0);
+    static_assert(LOADS <= 63, "vmcnt field");
     static_assert(STAGE % 16 == 0, "16-byte stages");
 };
 
@@ -93,6 +96,7 @@ __global__ __launch_bounds__(512) void strip_kernel(const StripArgs a) {
     constexpr int UPS = kTileK / UNIT, TB = S::TB, NT = S::NT, NR = S::NR;
     constexpr bool ALT2 = VAR == kVarGemv && WF != kStK16;
     constexpr bool ZP = BLK && WF != kStW8;
+    static_assert(U % 2 == 0, "the GEMV accumulator of a whole tile is its place in the stage");
     static_assert(!BLK || UNIT == 32, "K32 activation blocks");
     static_assert(BLK || WF == kStW4, "per-token mode: W4");
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -103,22 +107,39 @@ __global__ __launch_bounds__(512) void strip_kernel(const StripArgs a) {
     const int nblk = gridDim.x, id = blockIdx.x;
     const int q8 = nblk / 8, r8 = nblk % 8, xcd = id % 8, j8 = id / 8;
     const int L = xcd < r8 ? xcd * (q8 + 1) + j8 : r8 * (q8 + 1) + (xcd - r8) * q8 + j8;
-    int ei = 0;
+    // (the first entry and all four weights are read with constant indices,
+    // so their scalar loads go out together; an indexed read of the kernel
+    // arguments would add a dependent round trip each to the start)
+    StripEntry e = a.e[0];
     for (int i = 1; i < a.entries; ++i)
-        if (L >= a.e[i].blk) ei = i;
-    const int t0e = a.e[ei].t0, t1 = a.e[ei].t1, wi = a.e[ei].w;
-    const int within = L - a.e[ei].blk, ntt = (t1 - t0e + TT - 1) / TT;
-    const int t0 = t0e + within % ntt * TT;
-    const uint8_t *codes = a.w[wi].codes;
-    const uint8_t *scales = reinterpret_cast<const uint8_t *>(a.w[wi].scales);
-    const int M = a.w[wi].M, RG = M / 16;
+        if (L >= a.e[i].blk) e = a.e[i];
+    StripWeight w = a.w[0];
+#pragma unroll
+    for (int i = 1; i < kMaxWeights; ++i) {
+        StripWeight o = a.w[i];
+        asm volatile("" : "+s"(o.codes), "+s"(o.scales), "+s"(o.y), "+s"(o.M));
+        if (e.w == i) w = o;
+    }
+    const int t1 = e.t1;
+    const int within = L - e.blk, ntt = (t1 - e.t0 + TT - 1) / TT;
+    const int rgi = ntt == 1 ? within : within / ntt;        // (one token tile: no division)
+    const int t0 = e.t0 + (within - rgi * ntt) * TT;
+    const uint8_t *codes = w.codes;
+    const uint8_t *scales = reinterpret_cast<const uint8_t *>(w.scales);
+    const int M = w.M, RG = M / 16;
     const int K = a.K, NTK = K / kTileK, Nu = K / UNIT;
-    const int SP = a.S, SW = a.SW;
+    // streams of this block's entry: its splits, a.waves / RW at most (then
+    // each takes two in turn); with one row wave the waves left over take
+    // further row-groups (`item`), so entries of different split counts share
+    // a launch
+    const int SP = e.S, SW = min(SP, a.waves / RW);          // (powers of two)
+    const int ls = __builtin_ctz(SP), lsw = __builtin_ctz(SW);
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g4 = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int rw = wave % RW, sw = wave / RW;                // row wave, stream
-    const int rg = within / ntt * RW + rw;
+    const int rw = wave % RW, sw = RW == 1 ? wave & (SW - 1) : wave / RW;   // row wave, stream
+    const int item = RW == 1 ? wave >> lsw : 0;
+    const int rg = RW == 1 ? rgi * (a.waves >> lsw) + item : rgi * RW + rw;
     const int rgc = min(rg, RG - 1);                         // (row-groups past M load the last one, store nothing)
     const int gpt = kTileK / a.group;                        // scale groups per tile
     const int gsh = BLK && WF != kStK16 ? __builtin_ctz(a.group / 32) : 0;
@@ -149,7 +170,7 @@ __global__ __launch_bounds__(512) void strip_kernel(const StripArgs a) {
     const int sgr = gpt * 2;                                 // 16-byte pieces of scales per tile
     const uint8_t *const wrow = codes + (size_t)rgc * NTK * (kTileBytes * TB);
     const uint8_t *const srow = scales + (size_t)rgc * NTK * gpt * 32;
-    uint8_t *const ring = smem + sw * 2 * S::STAGE;
+    uint8_t *const ring = smem + (RW == 1 ? wave : sw) * 2 * S::STAGE;
     const uint8_t *wp = nullptr, *sp_ = nullptr, *qp = nullptr, *ap = nullptr;
     int islot = 0;                                           // stage the next issue fills
     auto seek = [&](int kt) {
@@ -212,9 +233,25 @@ __global__ __launch_bounds__(512) void strip_kernel(const StripArgs a) {
     const int s_rd = S::S_OFF + rw * S::S_ROW + n * 2;
     const int as_rd = S::AS_OFF + (TT >= 16 ? 4 * g4 : TT == 8 ? 4 * (g4 & 1) : 0) * 16;   // tokens of register 0
 
-    float res[NT][4] = {}, res_prev[NT][4];                       // this turn's chains and the turn before's
-    const int turns = SP / SW;                               // splits a stream runs in turn (1 or 2)
-    const int ls = __builtin_ctz(SP);
+    // The output's token scales and residuals, loaded where their latency
+    // hides: behind the first stage's loads (one row wave), else after the
+    // stream, before the split sum.
+    const int row = rg * 16 + n;
+    float tsc[NT][4], rsd[NT][4];
+    auto load_epilogue = [&]() {
+        if (sw != 0) return;
+#pragma unroll
+        for (int b = 0; b < NT; ++b)
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                const int t = min(t0 + 16 * b + 4 * g4 + r, t1 - 1);
+                if constexpr (!BLK) tsc[b][r] = a.ascale[t];
+                if (a.residual) rsd[b][r] = a.residual[(size_t)t * M + min(row, M - 1)];
+            }
+    };
+
+    float res[NT][4] = {}, res_prev[NT][4];                  // this turn's chains and the turn before's
+    const int turns = SP >> lsw;                             // splits a stream runs in turn (1 or 2)
 #pragma unroll 1
     for (int turn = 0; turn < turns; ++turn) {
         const int sp = sw * turns + turn;
@@ -241,6 +278,12 @@ __global__ __launch_bounds__(512) void strip_kernel(const StripArgs a) {
         seek(kt0);
         const int room = NTK - kt0;                          // tiles from the split's start to the end of K
         if (nst > 0) issue(room);
+        if (NT == 1 && RW == 1 && turn == 0) load_epilogue();           // (behind the first stage's loads)
+        // (a stream of two stages has both in flight from the start; longer
+        // ones keep one ahead: two cost more than they hide, T = 1, N = 5120,
+        // K = 17408 per-token 12.3 against 10.8 us)
+        const bool both = RW == 1 && nst == 2;
+        if (both) issue(room - U);
         // stages whose tiles lie wholly inside the split
         const int nfull = u0 % UPS == 0 && u1 % UPS == 0 ? ntl / U : 0;
 
@@ -281,20 +324,16 @@ __global__ __launch_bounds__(512) void strip_kernel(const StripArgs a) {
                         } else {
                             acc = mfma_k64(A[b][j], b0, zero);
                         }
-                        // (GEMV: units of odd index feed the second accumulator;
-                        // a split that starts on one swaps their roles, and
-                        // their sum commutes)
-                        const bool odd = ALT2 && (UNIT == 128 ? (kt & 1) : (j & 1));
+                        // GEMV: units at odd offsets from the split's start
+                        // feed the second accumulator. Stages hold an even
+                        // number of tiles, so a whole tile's parity is its
+                        // place in the stage; a split that starts on an odd
+                        // half tile swaps the two, and their sum commutes.
+                        constexpr bool kOddTile = UNIT == 128 && (UI & 1);
 #pragma unroll
                         for (int r = 0; r < NR; ++r) {
-                            if constexpr (ALT2 && UNIT == 128) {
-                                const float v = __builtin_fmaf((float)acc[r], ws, odd ? f1[b][r] : f0[b][r]);
-                                f0[b][r] = odd ? f0[b][r] : v;
-                                f1[b][r] = odd ? v : f1[b][r];
-                            } else {
-                                float &F = odd ? f1[b][r] : f0[b][r];
-                                F = __builtin_fmaf((float)acc[r], ws, F);
-                            }
+                            float &F = ALT2 && (kOddTile || (UNIT == 64 && j == 1)) ? f1[b][r] : f0[b][r];
+                            F = __builtin_fmaf((float)acc[r], ws, F);
                         }
                     }
                 }
@@ -376,7 +415,11 @@ __global__ __launch_bounds__(512) void strip_kernel(const StripArgs a) {
             }
         };
         for (int i = 0; i < nmax; ++i) {
-            KXW4_WAIT_VMCNT(0);                              // this wave's loads of stage i
+            // This wave's loads of stage i. Several row waves: the barrier
+            // publishes every wave's and frees the other stage; one: a
+            // stream's stages are its own.
+            if (both && i == 0) KXW4_WAIT_VMCNT(S::LOADS);
+            else KXW4_WAIT_VMCNT(0);
             if constexpr (RW > 1) {
                 lds_sync_after_dma();
             } else {
@@ -384,7 +427,7 @@ __global__ __launch_bounds__(512) void strip_kernel(const StripArgs a) {
                 __builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0): the reads of the stage refilled next
                 asm volatile("" ::: "memory");
             }
-            if (i + 1 < nst) issue(room - (i + 1) * U);
+            if (!both && i + 1 < nst) issue(room - (i + 1) * U);
             auto tiles = [&](auto edge) {
                 constexpr bool EDGE = decltype(edge)::value;
                 auto one = [&](auto uc) {
@@ -411,64 +454,94 @@ __global__ __launch_bounds__(512) void strip_kernel(const StripArgs a) {
             }
     }
 
+    if constexpr (NT > 1 || RW > 1) load_epilogue();
+
     // ---- ordered split sum (from 0.0f), then the output ----
     if (SP > 1) {
         float *part = reinterpret_cast<float *>(smem);
         lds_sync();                                          // every wave is past its last step
-        const int last = sw * turns + turns - 1;             // the wave's last split, in res
+        const int last = item * SP + sw * turns + turns - 1; // the wave's last split, in res
+        constexpr int PITCH = RW * NT * 256;                 // floats of one split
 #pragma unroll
         for (int b = 0; b < NT; ++b)
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
-                float *p = part + ((last * RW + rw) * NT + b) * 256 + r * 64 + lane;
+                float *p = part + last * PITCH + (rw * NT + b) * 256 + r * 64 + lane;
                 *p = res[b][r];
-                if (turns > 1) p[-RW * NT * 256] = res_prev[b][r];
+                if (turns > 1) p[-PITCH] = res_prev[b][r];
             }
         lds_sync();
         if (sw != 0) return;
+        // (all of a token block's partials are read before the ordered adds:
+        // a loop over the splits would wait for each read in turn)
+        auto split_sum = [&](auto sc) {
+            constexpr int SC = decltype(sc)::value;
 #pragma unroll
-        for (int b = 0; b < NT; ++b)
+            for (int b = 0; b < NT; ++b) {
+                float v[SC][4];
+                const float *p = part + item * SC * PITCH + (rw * NT + b) * 256 + lane;
 #pragma unroll
-            for (int r = 0; r < NR; ++r) {
-                const float *p = part + (rw * NT + b) * 256 + r * 64 + lane;
-                float sum = 0.0f;
-                for (int sp = 0; sp < SP; ++sp) sum = sum + p[sp * RW * NT * 256];
-                res[b][r] = sum;
+                for (int q = 0; q < SC; ++q)
+#pragma unroll
+                    for (int r = 0; r < NR; ++r) v[q][r] = p[q * PITCH + r * 64];
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    float sum = 0.0f;
+#pragma unroll
+                    for (int q = 0; q < SC; ++q) sum = sum + v[q][r];
+                    res[b][r] = sum;
+                }
             }
+        };
+        switch (SP) {
+        case 2: split_sum(std::integral_constant<int, 2>{}); break;
+        case 4: split_sum(std::integral_constant<int, 4>{}); break;
+        case 8: split_sum(std::integral_constant<int, 8>{}); break;
+        default: split_sum(std::integral_constant<int, 16>{}); break;
+        }
     }
     if (rg >= RG) return;
     constexpr float kInv16 = !BLK ? 0.0625f : 1.0f;          // the 16 w unpack's factor (per-token mode)
-    const int row = rg * 16 + n;
 #pragma unroll
     for (int b = 0; b < NT; ++b)
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
             const int tl = 16 * b + 4 * g4 + r, t = t0 + tl;
             if (t >= t1 || (TT < 16 && tl >= TT)) continue;
-            const float v = BLK ? res[b][r] : res[b][r] * (a.ascale[t] * kInv16);
+            const float v = BLK ? res[b][r] : res[b][r] * (tsc[b][r] * kInv16);
             float out;
-            if (a.residual) out = v + a.residual[(size_t)t * M + row];
+            if (a.residual) out = v + rsd[b][r];
             else if (VAR == kVarGemv && SP > 1) out = v + 0.0f;
             else out = v;
-            if (a.y_bf16) static_cast<uint16_t *>(a.w[wi].y)[(size_t)t * M + row] = float_to_bf16(out);
-            else static_cast<float *>(a.w[wi].y)[(size_t)t * M + row] = out;
+            if (a.y_bf16) static_cast<uint16_t *>(w.y)[(size_t)t * M + row] = float_to_bf16(out);
+            else static_cast<float *>(w.y)[(size_t)t * M + row] = out;
         }
 }
 
 template <int TT, int RW, int U, int UNIT, bool BLK, int VAR, int WF>
 static int st_launch(StripArgs &a, hipStream_t st) {
     using S = StShape<TT, RW, U, BLK, WF>;
-    int blk = 0;
-    for (int i = 0; i < a.entries; ++i) {
-        a.e[i].blk = blk;
-        blk += ((a.e[i].t1 - a.e[i].t0 + TT - 1) / TT) * ((a.w[a.e[i].w].M / 16 + RW - 1) / RW);
-    }
+    int smax = 1;
+    for (int i = 0; i < a.entries; ++i) smax = std::max(smax, a.e[i].S);
+    a.waves = RW > 1 ? smax * RW : a.same_s ? std::min(smax, 8) : smax >= 8 ? 8 : 4;
+    auto blocks = [&]() {
+        int blk = 0;
+        for (int i = 0; i < a.entries; ++i) {
+            a.e[i].blk = blk;
+            const int rows = RW == 1 ? a.waves / std::min(a.e[i].S, a.waves) : RW;   // row-groups per block
+            blk += ((a.e[i].t1 - a.e[i].t0 + TT - 1) / TT) * ((a.w[a.e[i].w].M / 16 + rows - 1) / rows);
+        }
+        return blk;
+    };
+    int blk = blocks();
     // Eight streams while every work-group is resident at once, else four
     // that take their splits in turn.
-    if (a.S == 8 && blk > device_cus() * (160 * 1024 / (16 * S::STAGE))) a.SW = 4;
-    const size_t part = a.S > 1 ? (size_t)a.S * RW * S::NT * 1024 : 0;
-    const size_t lds = std::max((size_t)2 * a.SW * S::STAGE, part);
-    if (lds > 160 * 1024 || a.SW * RW > 8) return -2;        // (the rules above never ask for it)
+    if (RW == 1 && smax == 8 && blk > device_cus() * (160 * 1024 / (16 * S::STAGE))) {
+        a.waves = 4;
+        blk = blocks();
+    }
+    const size_t lds = std::max((size_t)2 * (RW == 1 ? a.waves : smax) * S::STAGE, (size_t)std::max(2 * a.waves, RW) * S::NT * 1024);
+    if (lds > 160 * 1024 || a.waves > 8) return -2;          // (the rules below never ask for it)
     auto k = strip_kernel<TT, RW, U, UNIT, BLK, VAR, WF>;
     static bool attr[64] = {};                               // (the attribute is per device)
     int dev = 0;
@@ -479,7 +552,7 @@ static int st_launch(StripArgs &a, hipStream_t st) {
             return -6;
         attr[dev] = true;
     }
-    hipLaunchKernelGGL(k, dim3(blk), dim3(64 * a.SW * RW), lds, st, a);
+    hipLaunchKernelGGL(k, dim3(blk), dim3(64 * a.waves), lds, st, a);
     return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 
@@ -493,11 +566,11 @@ static int st_launch(StripArgs &a, hipStream_t st) {
 // us per-token and 22.2 against 24.4 us in block mode for two), two for W8
 // past 16 tokens, whose tiles are twice as large (T = 48: 37.0 against 46 us).
 template <int TT, int UNIT, bool BLK, int VAR, int WF>
-static int st_rw(StripArgs &a, int T, hipStream_t st) {
+static int st_rw(StripArgs &a, int T, int smax, hipStream_t st) {
     if constexpr (TT == 32) {
-        return a.S <= 2 ? st_launch<TT, 4, 2, UNIT, BLK, VAR, WF>(a, st) : st_launch<TT, 2, 2, UNIT, BLK, VAR, WF>(a, st);
+        return smax <= 2 ? st_launch<TT, 4, 2, UNIT, BLK, VAR, WF>(a, st) : st_launch<TT, 2, 2, UNIT, BLK, VAR, WF>(a, st);
     } else {
-        if (a.S == 1) {
+        if (smax == 1) {
             if constexpr (TT == 16) {
                 long long blks = 0;
                 for (int i = 0; i < a.entries; ++i)
@@ -507,7 +580,7 @@ static int st_rw(StripArgs &a, int T, hipStream_t st) {
             return st_launch<TT, 4, 2, UNIT, BLK, VAR, WF>(a, st);
         }
         if constexpr (TT == 16 && WF == kStW8) {
-            if (a.S <= 4 && T > 16) return st_launch<TT, 2, 2, UNIT, BLK, VAR, WF>(a, st);
+            if (smax <= 4 && a.same_s && T > 16) return st_launch<TT, 2, 2, UNIT, BLK, VAR, WF>(a, st);
         }
         return st_launch<TT, 1, 2, UNIT, BLK, VAR, WF>(a, st);
     }
@@ -515,11 +588,14 @@ static int st_rw(StripArgs &a, int T, hipStream_t st) {
 
 template <int UNIT, bool BLK, int VAR, int WF>
 static int st_shape(StripArgs &a, hipStream_t st) {
-    int T = 0;
+    int T = 0, smax = 1;
     long long strips16 = 0, strips32 = 0;
+    a.same_s = 1;
     for (int i = 0; i < a.entries; ++i) {
         const int t = a.e[i].t1 - a.e[i].t0, rgs = a.w[a.e[i].w].M / 16;
         T = std::max(T, t);
+        smax = std::max(smax, a.e[i].S);
+        a.same_s &= a.e[i].S == a.e[0].S;
         strips16 += (long long)rgs * ((t + 15) / 16);
         strips32 += (long long)rgs * ((t + 31) / 32);
     }
@@ -528,12 +604,12 @@ static int st_shape(StripArgs &a, hipStream_t st) {
     // (W8, with no unpack but twice the weight bytes: twice) and their
     // padding costs less than that (a 32-token strip takes 1.6 times a
     // 16-token one)
-    if (a.S <= 4 && strips16 * a.S > (WF == kStW8 ? 2000 : 4400) && 5 * strips16 > 8 * strips32)
-        return st_rw<32, UNIT, BLK, VAR, WF>(a, T, st);
-    if (T == 1) return st_rw<1, UNIT, BLK, VAR, WF>(a, T, st);
-    if (T == 2) return st_rw<2, UNIT, BLK, VAR, WF>(a, T, st);
-    if (T <= 8) return st_rw<8, UNIT, BLK, VAR, WF>(a, T, st);
-    return st_rw<16, UNIT, BLK, VAR, WF>(a, T, st);
+    if (smax <= 4 && a.same_s && strips16 * smax > (WF == kStW8 ? 2000 : 4400) && 5 * strips16 > 8 * strips32)
+        return st_rw<32, UNIT, BLK, VAR, WF>(a, T, smax, st);
+    if (T == 1) return st_rw<1, UNIT, BLK, VAR, WF>(a, T, smax, st);
+    if (T == 2) return st_rw<2, UNIT, BLK, VAR, WF>(a, T, smax, st);
+    if (T <= 8) return st_rw<8, UNIT, BLK, VAR, WF>(a, T, smax, st);
+    return st_rw<16, UNIT, BLK, VAR, WF>(a, T, smax, st);
 }
 
 bool strip_takes(int group, int block, int scale_enc, long long T, int K) {
@@ -542,7 +618,6 @@ bool strip_takes(int group, int block, int scale_enc, long long T, int K) {
 }
 
 int launch_strip(StripArgs &a, hipStream_t st) {
-    a.SW = std::min(a.S, 8);
     if (a.scale_enc == 2)
         return a.variant == kVarGemv ? st_shape<32, true, kVarGemv, kStW8>(a, st) : st_shape<32, true, kVarGemm, kStW8>(a, st);
     if (a.group == 16) return st_shape<32, true, kVarGemv, kStK16>(a, st);
@@ -555,19 +630,6 @@ int launch_strip(StripArgs &a, hipStream_t st) {
     if (a.group == 128)
         return a.variant == kVarGemv ? st_shape<128, false, kVarGemv, kStW4>(a, st) : st_shape<128, false, kVarGemm, kStW4>(a, st);
     return a.variant == kVarGemv ? st_shape<64, false, kVarGemv, kStW4>(a, st) : st_shape<64, false, kVarGemm, kStW4>(a, st);
-}
-
-int launch_strip_classes(const DecodeArgs &a, hipStream_t st) {
-    int seen = 0;                                            // the split counts are powers of two
-    for (int i = 0; i < a.count; ++i)
-        for (int g = 0; g < a.seg_count; ++g) seen |= a.w[i].seg_split[g];
-    for (int S = 16; S >= 1; S >>= 1) {
-        if (!(seen & S)) continue;
-        StripArgs s = strip_args(a, a.variant, S);
-        const int r = launch_strip(s, st);
-        if (r) return r;
-    }
-    return 0;
 }
 
 }  // namespace kxw4
