@@ -11,6 +11,8 @@
 #include "kxw4_device.hpp"
 #include "kxw4_internal.hpp"
 
+#include <algorithm>
+
 namespace kxw4 {
 
 // Tile-local coordinates of packed dword `d` (0..255 within a tile).
@@ -110,43 +112,102 @@ __global__ void import_ref_codes_kernel(const uint8_t *__restrict__ ref, int M, 
 }
 
 // ---- E2M3 -> asymmetric int4 (kernels_dpas.cpp:49-69, 229-344) -----------
+//
+// One thread per (row, group), the 16 rows of a row-group fastest, then the
+// groups: a wave covers 16 rows x 4 groups, whose payload, codes and scales
+// are contiguous. What bounds it is the fit's arithmetic, four quotients per
+// weight (three refinements and the codes), not memory: 89 M weights (K =
+// 5120, M = 17408, group 32) move 117 MB, 24 us at the rate a large copy
+// reaches. With a byte load or two per code and an IEEE division per quotient
+// (about 12 instructions) it took 215 us; with three 16-byte loads per thread,
+// quotients of five operations and coalesced stores 107 us (W8, M = 7408, K =
+// 2048: 39 -> 15 us).
 
+// Six-bit code as a float: the five magnitude bits are the exponent and
+// mantissa of an E2M3 number, put where FP32's lie and scaled by 2^126 (an
+// exponent field of 0 is subnormal in both formats, so the product is exact).
 __device__ __forceinline__ float e2m3f(uint32_t c) {
-    const float m = (float)(c & 7u);
-    const uint32_t e = (c >> 3) & 3u;
-    const float v = (e == 0) ? m * 0.125f : (1.0f + m * 0.125f) * (float)(1u << (e - 1));
-    return (c & 0x20u) ? -v : v;
+    const float v = __uint_as_float((c & 0x1Fu) << 20) * __uint_as_float(0x7E800000u);
+    return __uint_as_float(__float_as_uint(v) | ((c & 0x20u) << 26));
 }
 
-__device__ __forceinline__ uint32_t e2m3_code_at(const uint8_t *__restrict__ payload, int Kt,
-                                                 int row, int col) {
-    const int mt = row >> 4;
-    const int kt = col >> 5;
-    const int lane = (((row & 15) >> 1) << 2) | ((col & 31) >> 3);
-    const int idx = (((col >> 2) & 1) << 3) | ((row & 1) << 2) | (col & 3);
-    const int bit = 6 * idx;
-    const uint8_t *p = payload + ((size_t)mt * Kt + kt) * 384u + (size_t)lane * 12u;
-    uint32_t bits = p[bit >> 3];
-    if ((bit & 7) > 2) bits |= (uint32_t)p[(bit >> 3) + 1] << 8;
-    return (bits >> (bit & 7)) & 0x3fu;
+// The 32 codes of (row, K32 tile): lanes 4*(row%16/2) .. +3 of the tile's 384
+// bytes, 12 bytes each holding eight columns of an even and an odd row as a
+// 96-bit stream (codes 0-3 even, 4-7 odd, 8-11 even, 12-15 odd).
+__device__ __forceinline__ void e2m3_unit(const uint8_t *__restrict__ payload, size_t tile, int n, float b,
+                                          float *wf) {
+    const uint8_t *src = payload + tile * 384u + (size_t)(n >> 1) * 48u;
+    uint32_t w[12] = {};
+    if ((reinterpret_cast<uintptr_t>(payload) & 15) == 0) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const v4u v = reinterpret_cast<const v4u *>(src)[i];
+            w[4 * i] = v.x;
+            w[4 * i + 1] = v.y;
+            w[4 * i + 2] = v.z;
+            w[4 * i + 3] = v.w;
+        }
+    } else {                                                 // (a payload that starts anywhere)
+#pragma unroll
+        for (int i = 0; i < 48; ++i) w[i >> 2] |= (uint32_t)src[i] << (8 * (i & 3));
+    }
+    const bool odd = n & 1;
+#pragma unroll
+    for (int l = 0; l < 4; ++l) {
+        const uint32_t x = w[3 * l], y = w[3 * l + 1], z = w[3 * l + 2];
+        const uint32_t first = odd ? (x >> 24) | (y << 8) : x;
+        const uint32_t second = odd ? z >> 8 : (y >> 16) | (z << 16);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            wf[8 * l + i] = e2m3f(first >> (6 * i)) * b;
+            wf[8 * l + 4 + i] = e2m3f(second >> (6 * i)) * b;
+        }
+    }
+}
+
+// a / s in round to nearest. SAFE: the two-step refinement of a * y with
+// y = fl(1/s) (Markstein: from a faithful quotient q and a correctly rounded
+// reciprocal, fl(q + fl(a - q s) y) is the correctly rounded quotient, the
+// remainder being exact), for operands far from the ends of the range.
+template <bool SAFE>
+__device__ __forceinline__ float quot(float a, float s, float y) {
+    if constexpr (!SAFE) return a / s;
+    float q = a * y;
+    q = __builtin_fmaf(__builtin_fmaf(-q, s, a), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-q, s, a), y, q);
+}
+
+// Block scales this far from the ends of the range keep every weight, fitted
+// scale, quotient and remainder normal (the scales lie in [b/120, 8b], or are
+// 1 where every weight is 0; the FP16 scale is checked by itself).
+__device__ __forceinline__ bool safe_scale(float b) { return b > 0x1p-60f && b < 0x1p60f; }
+__device__ __forceinline__ bool safe_half(float s) { return s > 0.0f && s < 65536.0f; }
+
+// min(max(x, lo), hi) of a number that is not NaN (clampf's result then)
+template <bool SAFE>
+__device__ __forceinline__ float clampq(float x, float lo, float hi) {
+    return SAFE ? __builtin_amdgcn_fmed3f(x, lo, hi) : clampf(x, lo, hi);
 }
 
 // fit_int4_asym with the least-squares sums evaluated as fused multiply-adds.
-template <int N>
-__device__ uint16_t fit_int4_asym(const float *wf, int *out_z) {
+template <int N, bool SAFE>
+__device__ __forceinline__ uint16_t fit_int4_asym(const float *wf, int *out_z) {
     float lo = 0.0f, hi = 0.0f;
+#pragma unroll
     for (int j = 0; j < N; ++j) {
         lo = fminf(lo, wf[j]);
         hi = fmaxf(hi, wf[j]);
     }
     float s = (hi - lo) / 15.0f;
     if (!(s > 0.0f)) s = 1.0f;
+#pragma unroll 1
     for (int iter = 0; iter < 3; ++iter) {
-        const int zi = (int)clampf(rintf(-lo / s) - 8.0f, -8.0f, 7.0f);
+        const float zf = (float)(int)clampf(rintf(-lo / s) - 8.0f, -8.0f, 7.0f), y = 1.0f / s;
         float num = 0.0f, den = 0.0f;
+#pragma unroll
         for (int j = 0; j < N; ++j) {
-            const float q = clampf(rintf(wf[j] / s + (float)zi), -8.0f, 7.0f);
-            const float c = q - (float)zi;
+            const float q = clampq<SAFE>(rintf(quot<SAFE>(wf[j], s, y) + zf), -8.0f, 7.0f);
+            const float c = q - zf;
             num = __builtin_fmaf(wf[j], c, num);
             den = __builtin_fmaf(c, c, den);
         }
@@ -158,54 +219,72 @@ __device__ uint16_t fit_int4_asym(const float *wf, int *out_z) {
     return sh;
 }
 
-// One thread per (row, group): decode, fit, then write the group's packed
-// dwords (a group of 32 or 64 K owns whole dwords in every lane group) and
-// its FP16|zp scale.
-template <int GROUP>
-__global__ void repack_e2m3_kernel(const uint8_t *__restrict__ payload,
-                                   const float *__restrict__ bs, int scale_cols, int M, int K,
-                                   uint32_t *__restrict__ out_codes,
-                                   uint16_t *__restrict__ out_scales) {
-    const int G = K / GROUP, Kt = K / 32, NT = K / kTileK;
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)M * G) return;
-    const int row = (int)(i / G), g = (int)(i % G);
-    const int mt = row >> 4;
-    const int k0 = g * GROUP;
-    float wf[GROUP];
-#pragma unroll
-    for (int j = 0; j < GROUP; ++j) {
-        const int kt = (k0 + j) >> 5;
-        const int sc = (scale_cols == Kt) ? kt : (kt >> 2);
-        const float b = bs[(size_t)(mt >> 3) * scale_cols + sc];
-        wf[j] = e2m3f(e2m3_code_at(payload, Kt, row, k0 + j)) * b;
-    }
+// Fit N weights and return their scale word; their 4-bit codes go to q4.
+template <int N>
+__device__ __forceinline__ uint16_t quant_int4(const float *wf, bool safe, uint32_t *q4) {
     int z = 0;
-    const uint16_t sh = fit_int4_asym<GROUP>(wf, &z);
-    out_scales[((size_t)mt * G + g) * 16 + (row & 15)] = (uint16_t)(sh | (z & 0xF));
-    const float gs = half_bits_to_float(sh);
-    uint8_t q4[GROUP];
+    const uint16_t sh = safe ? fit_int4_asym<N, true>(wf, &z) : fit_int4_asym<N, false>(wf, &z);
+    const float gs = half_bits_to_float(sh), zf = (float)z;
+    if (safe && safe_half(gs)) {
+        const float y = 1.0f / gs;
 #pragma unroll
-    for (int j = 0; j < GROUP; ++j)
-        q4[j] = (uint8_t)((int)clampf(rintf(wf[j] / gs + (float)z), -8.0f, 7.0f) & 0xF);
-    // Dwords of this group: K32 unit u = (k0 + 32v) covers tile kb, dword
-    // i = (u % 128) / 32, for the four lane groups gl (k = 32i + 8gl + b).
-    const int n = row & 15;
+        for (int j = 0; j < N; ++j)
+            q4[j] = (uint32_t)(int)clampq<true>(rintf(quot<true>(wf[j], gs, y) + zf), -8.0f, 7.0f) & 0xFu;
+    } else {
 #pragma unroll
-    for (int v = 0; v < GROUP / 32; ++v) {
-        const int k = k0 + 32 * v;
-        const int kb = k / kTileK, di = (k % kTileK) / 32;
-        uint32_t *tile = out_codes + ((size_t)mt * NT + kb) * 256;
+        for (int j = 0; j < N; ++j) q4[j] = (uint32_t)(int)clampf(rintf(wf[j] / gs + zf), -8.0f, 7.0f) & 0xFu;
+    }
+    return (uint16_t)(sh | (z & 0xF));
+}
+
+// The four packed dwords of one K32 unit of a row: dword u of lane groups
+// gl = 0..3 (k = 32u + 8gl + b, b = 0..3 low nibbles, 4..7 high).
+__device__ __forceinline__ void store_unit(uint32_t *__restrict__ tile, int n, int u, const uint32_t *q4) {
 #pragma unroll
-        for (int gl = 0; gl < 4; ++gl) {
-            uint32_t w = 0;
+    for (int gl = 0; gl < 4; ++gl) {
+        uint32_t w = 0;
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const int j = 32 * v + 8 * gl + b;
-                w |= ((uint32_t)q4[j] | ((uint32_t)q4[j + 4] << 4)) << (8 * b);
-            }
-            tile[(n + 16 * gl) * 4 + di] = w;
-        }
+        for (int b = 0; b < 4; ++b) w |= (q4[8 * gl + b] | (q4[8 * gl + b + 4] << 4)) << (8 * b);
+        tile[(n + 16 * gl) * 4 + u] = w;
+    }
+}
+
+// GROUP 32 or 64: a thread's group is one or two whole K32 units. GROUP 16
+// (mode 1, the K16 tier, kernels_dpas.cpp:287-296): a thread fits the two
+// halves of one K32 unit.
+template <int GROUP>
+__global__ __launch_bounds__(256) void repack_e2m3_kernel(const uint8_t *__restrict__ payload,
+                                                          const float *__restrict__ bs, int scale_cols, int M, int K,
+                                                          uint32_t *__restrict__ out_codes,
+                                                          uint16_t *__restrict__ out_scales) {
+    constexpr int SPAN = GROUP < 32 ? 32 : GROUP, UNITS = SPAN / 32;
+    const int SG = K / SPAN, Kt = K / 32, NT = K / kTileK;
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (size_t)M * SG) return;
+    const int n = (int)(i & 15);
+    const size_t rgg = i >> 4;                               // row-group * SG + span
+    const int mt = (int)(rgg / SG), g = (int)(rgg - (size_t)mt * SG);
+    float wf[SPAN];
+    bool safe = true;
+#pragma unroll
+    for (int v = 0; v < UNITS; ++v) {
+        const int kt = g * UNITS + v;
+        const float b = bs[(size_t)(mt >> 3) * scale_cols + (scale_cols == Kt ? kt : kt >> 2)];
+        safe = safe && safe_scale(b);
+        e2m3_unit(payload, (size_t)mt * Kt + kt, n, b, wf + 32 * v);
+    }
+    uint32_t q4[SPAN];
+    if constexpr (GROUP < 32) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            out_scales[((size_t)mt * 2 * Kt + 2 * g + h) * 16 + n] = quant_int4<16>(wf + 16 * h, safe, q4 + 16 * h);
+    } else {
+        out_scales[((size_t)mt * SG + g) * 16 + n] = quant_int4<GROUP>(wf, safe, q4);
+    }
+#pragma unroll
+    for (int v = 0; v < UNITS; ++v) {
+        const int kt = g * UNITS + v;
+        store_unit(out_codes + ((size_t)mt * NT + (kt >> 2)) * 256, n, kt & 3, q4 + 32 * v);
     }
 }
 
@@ -252,18 +331,23 @@ __global__ void unpack_s8_kernel(const uint32_t *__restrict__ in, int M, int K, 
 
 // w8_repack_kernel's fit with the least-squares sums as fused multiply-adds:
 // s = max(hi/127, neg/128), two refinements, FP16 by round to nearest even.
-__device__ uint16_t fit_int8(const float *wf) {
+template <bool SAFE>
+__device__ __forceinline__ uint16_t fit_int8(const float *wf) {
     float hi = 0.0f, neg = 0.0f;
+#pragma unroll
     for (int j = 0; j < 32; ++j) {
         hi = fmaxf(hi, wf[j]);
         neg = fmaxf(neg, -wf[j]);
     }
     float s = fmaxf(hi / 127.0f, neg / 128.0f);
     if (!(s > 0.0f)) s = 1.0f;
+#pragma unroll 1
     for (int iter = 0; iter < 2; ++iter) {
+        const float y = 1.0f / s;
         float num = 0.0f, den = 0.0f;
+#pragma unroll
         for (int j = 0; j < 32; ++j) {
-            const float q = clampf(rintf(wf[j] / s), -128.0f, 127.0f);
+            const float q = clampq<SAFE>(rintf(quot<SAFE>(wf[j], s, y)), -128.0f, 127.0f);
             num = __builtin_fmaf(wf[j], q, num);
             den = __builtin_fmaf(q, q, den);
         }
@@ -272,76 +356,45 @@ __device__ uint16_t fit_int8(const float *wf) {
     return __builtin_bit_cast(uint16_t, (_Float16)s);
 }
 
-// One thread per (row, K32): decode, fit, write the unit's 8 dwords (two per
-// lane group) and its tiled FP16 scale.
-__global__ void repack_e2m3_s8_kernel(const uint8_t *__restrict__ payload, const float *__restrict__ bs,
-                                      int scale_cols, int M, int K, uint32_t *__restrict__ out_codes,
-                                      uint16_t *__restrict__ out_scales) {
+// One thread per (row, K32), rows of a row-group fastest (as the int4 repack
+// above, which says what bounds it): decode, fit, write the unit's 8 dwords
+// (two per lane group, one 8-byte store) and its tiled FP16 scale.
+__global__ __launch_bounds__(256) void repack_e2m3_s8_kernel(const uint8_t *__restrict__ payload,
+                                                             const float *__restrict__ bs, int scale_cols, int M, int K,
+                                                             uint32_t *__restrict__ out_codes,
+                                                             uint16_t *__restrict__ out_scales) {
     const int Kt = K / 32, NT = K / kTileK;
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (size_t)M * Kt) return;
-    const int row = (int)(i / Kt), kt = (int)(i % Kt);
-    const int mt = row >> 4, n = row & 15;
-    const int sc = (scale_cols == Kt) ? kt : (kt >> 2);
-    const float b = bs[(size_t)(mt >> 3) * scale_cols + sc];
+    const int n = (int)(i & 15);
+    const size_t unit = i >> 4;                              // row-group * Kt + K32 tile
+    const int mt = (int)(unit / Kt), kt = (int)(unit - (size_t)mt * Kt);
+    const float b = bs[(size_t)(mt >> 3) * scale_cols + (scale_cols == Kt ? kt : kt >> 2)];
+    const bool safe = safe_scale(b);
     float wf[32];
-#pragma unroll
-    for (int j = 0; j < 32; ++j) wf[j] = e2m3f(e2m3_code_at(payload, Kt, row, kt * 32 + j)) * b;
-    const uint16_t sh = fit_int8(wf);
-    out_scales[((size_t)mt * Kt + kt) * 16 + n] = sh;
+    e2m3_unit(payload, unit, n, b, wf);
+    const uint16_t sh = safe ? fit_int8<true>(wf) : fit_int8<false>(wf);
+    out_scales[unit * 16 + n] = sh;
     const float st = half_bits_to_float(sh);
-    const int kb = kt >> 2, j = kt & 3;
-    uint32_t *tile = out_codes + ((size_t)mt * NT + kb) * 512 + 256 * (j >> 1);
+    uint32_t w[8] = {};
+    if (safe && safe_half(st)) {
+        const float y = 1.0f / st;
 #pragma unroll
-    for (int gl = 0; gl < 4; ++gl)
+        for (int j = 0; j < 32; ++j)
+            w[j >> 2] |= (uint32_t)(uint8_t)(int)clampq<true>(rintf(quot<true>(wf[j], st, y)), -128.0f, 127.0f) << (8 * (j & 3));
+    } else {
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            uint32_t w = 0;
-#pragma unroll
-            for (int bb = 0; bb < 4; ++bb) {
-                const int q = (int)clampf(rintf(wf[8 * gl + 4 * e + bb] / st), -128.0f, 127.0f);
-                w |= (uint32_t)(uint8_t)q << (8 * bb);
-            }
-            tile[(n + 16 * gl) * 4 + 2 * (j & 1) + e] = w;
-        }
-}
-
-// Mode 1, the K16 tier (kernels_dpas.cpp:287-296): one thread per (row, K32
-// tile) fits its two K16 halves (FP16|zp each); half h owns dword kt % 4 of
-// lane groups 2h and 2h + 1.
-__global__ void repack_e2m3_k16_kernel(const uint8_t *__restrict__ payload,
-                                       const float *__restrict__ bs, int scale_cols, int M, int K,
-                                       uint32_t *__restrict__ out_codes,
-                                       uint16_t *__restrict__ out_scales) {
-    const int Kt = K / 32, NT = K / kTileK, G = K / 16;
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)M * Kt) return;
-    const int row = (int)(i / Kt), kt = (int)(i % Kt);
-    const int mt = row >> 4, n = row & 15;
-    const int sc = (scale_cols == Kt) ? kt : (kt >> 2);
-    const float b = bs[(size_t)(mt >> 3) * scale_cols + sc];
-    float wf[32];
-#pragma unroll
-    for (int j = 0; j < 32; ++j) wf[j] = e2m3f(e2m3_code_at(payload, Kt, row, kt * 32 + j)) * b;
-    uint8_t q4[32];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        int z = 0;
-        const uint16_t sh = fit_int4_asym<16>(wf + 16 * h, &z);
-        out_scales[((size_t)mt * G + 2 * kt + h) * 16 + n] = (uint16_t)(sh | (z & 0xF));
-        const float gs = half_bits_to_float(sh);
-#pragma unroll
-        for (int j = 16 * h; j < 16 * h + 16; ++j)
-            q4[j] = (uint8_t)((int)clampf(rintf(wf[j] / gs + (float)z), -8.0f, 7.0f) & 0xF);
+        for (int j = 0; j < 32; ++j)
+            w[j >> 2] |= (uint32_t)(uint8_t)(int)clampf(rintf(wf[j] / st), -128.0f, 127.0f) << (8 * (j & 3));
     }
-    uint32_t *tile = out_codes + ((size_t)mt * NT + kt / 4) * 256;
+    const int j = kt & 3;
+    uint32_t *tile = out_codes + ((size_t)mt * NT + (kt >> 2)) * 512 + 256 * (j >> 1);
 #pragma unroll
     for (int gl = 0; gl < 4; ++gl) {
-        uint32_t w = 0;
-#pragma unroll
-        for (int bb = 0; bb < 4; ++bb)
-            w |= ((uint32_t)q4[8 * gl + bb] | ((uint32_t)q4[8 * gl + bb + 4] << 4)) << (8 * bb);
-        tile[(n + 16 * gl) * 4 + (kt & 3)] = w;
+        v2u o;
+        o.x = w[2 * gl];
+        o.y = w[2 * gl + 1];
+        *reinterpret_cast<v2u *>(tile + (n + 16 * gl) * 4 + 2 * (j & 1)) = o;
     }
 }
 
@@ -371,7 +424,7 @@ int launch_unpack_s8(const uint8_t *codes, const uint16_t *scales, int M, int K,
 int launch_repack_e2m3_s8(const uint8_t *payload, const float *bs, int scale_cols, int M, int K,
                           uint8_t *out_codes, uint16_t *out_scales, hipStream_t st) {
     const size_t n = (size_t)M * (K / 32);
-    hipLaunchKernelGGL(repack_e2m3_s8_kernel, dim3(blocks_for(n, 128)), dim3(128), 0, st, payload, bs,
+    hipLaunchKernelGGL(repack_e2m3_s8_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, st, payload, bs,
                        scale_cols, M, K, reinterpret_cast<uint32_t *>(out_codes), out_scales);
     return hipGetLastError() == hipSuccess ? 0 : -6;
 }
@@ -410,17 +463,10 @@ int launch_import_ref(const uint8_t *ref_codes, const uint16_t *ref_scales, int 
 
 int launch_repack_e2m3(const uint8_t *payload, const float *bs, int scale_cols, int M, int K,
                        int group, uint8_t *out_codes, uint16_t *out_scales, hipStream_t st) {
-    const size_t n = (size_t)M * (K / group);
-    uint32_t *oc = reinterpret_cast<uint32_t *>(out_codes);
-    if (group == 16)
-        hipLaunchKernelGGL(repack_e2m3_k16_kernel, dim3(blocks_for((size_t)M * (K / 32), 128)), dim3(128), 0,
-                           st, payload, bs, scale_cols, M, K, oc, out_scales);
-    else if (group == 32)
-        hipLaunchKernelGGL(repack_e2m3_kernel<32>, dim3(blocks_for(n, 128)), dim3(128), 0, st,
-                           payload, bs, scale_cols, M, K, oc, out_scales);
-    else
-        hipLaunchKernelGGL(repack_e2m3_kernel<64>, dim3(blocks_for(n, 128)), dim3(128), 0, st,
-                           payload, bs, scale_cols, M, K, oc, out_scales);
+    const size_t n = (size_t)M * (K / std::max(group, 32));
+    auto k = group == 16 ? repack_e2m3_kernel<16> : group == 32 ? repack_e2m3_kernel<32> : repack_e2m3_kernel<64>;
+    hipLaunchKernelGGL(k, dim3(blocks_for(n, 256)), dim3(256), 0, st, payload, bs, scale_cols, M, K,
+                       reinterpret_cast<uint32_t *>(out_codes), out_scales);
     return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 
