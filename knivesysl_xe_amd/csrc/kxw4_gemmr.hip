@@ -21,8 +21,9 @@
 // as possible to the chain:
 //   * weights are the MFMA's A operand and activations its B operand, so a
 //     lane holds one token and 16 rows of a block: the activation scale is
-//     one value per lane and unit, and the 16 weight scales (and the weight
-//     unpack) are shared by the wave's NT token blocks;
+//     one value per lane and unit, and the 16 weight scales (FP32, prepared
+//     once per stage) and the weight unpack are shared by the wave's NT
+//     token blocks;
 //   * a wave owns 32 rows x 32*NT tokens; a work-group WR x WT waves;
 //   * per 128-K step the activation tile (XOR-swizzled rows), the packed
 //     weight tiles, the FP16|zp scales and the activation scales of the
@@ -85,11 +86,11 @@ struct GrShape {
     static constexpr int W_OFF = A_BYTES;
     static constexpr int S_OFF = W_OFF + W_BYTES;
     static constexpr int AS_OFF = (S_OFF + S_BYTES + 15) / 16 * 16;
-    // prepared once per stage by the waves that loaded the scales: the FP16
-    // scales with the zero-point nibble cleared ([row-group][group][16]
-    // u16) and the zero-point bytes z + 8 ([row-group][group][16] u8)
+    // prepared once per stage by the waves that loaded the scales: the
+    // scales as FP32, the zero-point nibble cleared ([row-group][group][16]),
+    // and the zero-point bytes z + 8 ([row-group][group][16] u8)
     static constexpr int MS_OFF = AS_OFF + AS_BYTES;
-    static constexpr int ZZ_OFF = MS_OFF + S_BYTES;
+    static constexpr int ZZ_OFF = MS_OFF + 2 * S_BYTES;
     static constexpr int STAGE = (ZZ_OFF + S_BYTES / 2 + 1023) / 1024 * 1024;
     // loads per wave and stage, equal for every wave (one vmcnt retires a
     // stage); chunk indices wrap when the waves do not divide them, and a
@@ -219,7 +220,7 @@ __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemmr_kernel(const GemmArgs 
     const int zz_lds = S::ZZ_OFF + rgl * GPS * 16 + (m & 15);
     // weight scales of this lane's output rows 8q + 4kg + e (e = 0..3) of
     // the wave's row block: row-group 2wr + q/2, rows 8(q%2) + 4kg + e
-    const int ws_lds = (ZP ? S::MS_OFF : S::S_OFF) + 2 * wr * GPS * 32 + 8 * kg;   // + (q/2) GPS 32 + (q%2) 16
+    const int ws_lds = S::MS_OFF + 2 * wr * GPS * 64 + 16 * kg;   // + (q/2) GPS 64 + (q%2) 32
     // activation pieces of token block j: row tb + m, pieces 4c + 2kg + {0,1}
     const int tb = wt * NT * 32;                             // first token of this wave in the tile
     const int tsw = ((tb + m) >> 1) & 7;                     // the row's swizzle (tb is a multiple of 32)
@@ -248,29 +249,35 @@ __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemmr_kernel(const GemmArgs 
         else if (NST >= 3 && later >= 1) KXW4_WAIT_VMCNT(LD);
         else KXW4_WAIT_VMCNT(0);
         const uint8_t *sb = smem + st * STAGE;
-        if constexpr (ZP) {
-            // the scale granules this wave loaded into the stage (8 rows of
-            // one row-group and scale group each): masked scales and
-            // zero-point bytes, published by the barrier below (written to
-            // their own regions, so a granule two waves loaded is prepared
-            // twice with the same values)
-            if (lane < S::S_LANES) {
-                const int gi = (wave * S::S_LANES) % S::S_TOTAL + lane;
-                const v4u p = *reinterpret_cast<const v4u *>(sb + S::S_OFF + gi * 16);
-                v4u ms;
-                ms.x = p.x & 0xFFF0FFF0u;
-                ms.y = p.y & 0xFFF0FFF0u;
-                ms.z = p.z & 0xFFF0FFF0u;
-                ms.w = p.w & 0xFFF0FFF0u;
-                *reinterpret_cast<v4u *>(const_cast<uint8_t *>(sb) + S::MS_OFF + gi * 16) = ms;
+        // the scale granules this wave loaded into the stage (8 rows of one
+        // row-group and scale group each): FP32 scales and zero-point bytes,
+        // published by the barrier below (written to their own regions, so a
+        // granule two waves loaded is prepared twice with the same values)
+        if (lane < S::S_LANES) {
+            const int gi = (wave * S::S_LANES) % S::S_TOTAL + lane;
+            const v4u p = *reinterpret_cast<const v4u *>(sb + S::S_OFF + gi * 16);
+            constexpr uint32_t keep = ZP ? 0xFFF0u : 0xFFFFu;
+            v4f m0, m1;
+            m0.x = half_bits_to_float((uint16_t)(p.x & keep));
+            m0.y = half_bits_to_float((uint16_t)((p.x >> 16) & keep));
+            m0.z = half_bits_to_float((uint16_t)(p.y & keep));
+            m0.w = half_bits_to_float((uint16_t)((p.y >> 16) & keep));
+            m1.x = half_bits_to_float((uint16_t)(p.z & keep));
+            m1.y = half_bits_to_float((uint16_t)((p.z >> 16) & keep));
+            m1.z = half_bits_to_float((uint16_t)(p.w & keep));
+            m1.w = half_bits_to_float((uint16_t)((p.w >> 16) & keep));
+            v4f *ms = reinterpret_cast<v4f *>(const_cast<uint8_t *>(sb) + S::MS_OFF + gi * 32);
+            ms[0] = m0;
+            ms[1] = m1;
+            if constexpr (ZP) {
                 // z + 8 = (p & 15) ^ 8 of each row, one byte per row: bytes
                 // 0 and 2 of each dword pair up with the two rows it holds
-                uint2 zb;
+                v2u zb;
                 zb.x = __builtin_amdgcn_perm(p.y, p.x, 0x06040200u) & 0x0F0F0F0Fu;
                 zb.y = __builtin_amdgcn_perm(p.w, p.z, 0x06040200u) & 0x0F0F0F0Fu;
                 zb.x ^= 0x08080808u;
                 zb.y ^= 0x08080808u;
-                *reinterpret_cast<uint2 *>(const_cast<uint8_t *>(sb) + S::ZZ_OFF + gi * 8) = zb;
+                *reinterpret_cast<v2u *>(const_cast<uint8_t *>(sb) + S::ZZ_OFF + gi * 8) = zb;
             }
         }
         lds_sync_after_dma();
@@ -298,14 +305,14 @@ __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemmr_kernel(const GemmArgs 
 #pragma unroll
             for (int g = 0; g < GPS; ++g) zc[g] = zc_of(g);
         }
-        // FP16 scales of the 16 output rows of scale group g (the zero-point
-        // nibble cleared): dword r/2, half r%2 is register r's row
-        auto read_ws = [&](int g, uint32_t (&w)[8]) {
+        // scales of the 16 output rows of scale group g: register r's row is
+        // element r
+        auto read_ws = [&](int g, float (&w)[16]) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const v2u v = *reinterpret_cast<const v2u *>(sb + ws_lds + (q >> 1) * GPS * 32 + (q & 1) * 16 + g * 32);
-                w[2 * q] = v.x;
-                w[2 * q + 1] = v.y;
+                const v4f v = *reinterpret_cast<const v4f *>(sb + ws_lds + (q >> 1) * GPS * 64 + (q & 1) * 32 + g * 64);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) w[4 * q + e] = v[e];
             }
         };
         // item i's activation operand (this unit's 8 bytes of pieces
@@ -336,20 +343,12 @@ __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemmr_kernel(const GemmArgs 
         // instruction costs a wait state)
         // (two at a time in the lean pipeline, whose registers are short)
         constexpr int CHK = LEAN ? 2 : 4;
-        auto chain = [&](int j, const v16i &d, const uint32_t (&wsr)[8], float as) {
+        auto chain = [&](int j, const v16i &d, const float (&wsr)[16], float as) {
 #pragma unroll
             for (int r0 = 0; r0 < 16; r0 += CHK) {
                 float wa[CHK], pv[CHK];
 #pragma unroll
-                for (int e = 0; e < CHK; ++e) {
-                    const int r = r0 + e;
-                    const uint32_t wv = wsr[r >> 1];
-                    const float wsv = (float)__builtin_bit_cast(_Float16, (uint16_t)((r & 1) ? (wv >> 16) : wv));
-                    // ws * as rounded once: fma(ws, as, +0) equals the
-                    // product except for its zero sign, which the chain's
-                    // fma ignores (the accumulator is never -0)
-                    wa[e] = __builtin_fmaf(wsv, as, 0.0f);
-                }
+                for (int e = 0; e < CHK; ++e) wa[e] = wsr[r0 + e] * as;
 #pragma unroll
                 for (int e = 0; e < CHK; ++e) pv[e] = (float)d[r0 + e];
 #pragma unroll
@@ -362,7 +361,7 @@ __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemmr_kernel(const GemmArgs 
             // Few registers (more waves per SIMD hide the latencies): item
             // i + 1's operands are read during item i, and each item's
             // chain follows its own MFMA.
-            uint32_t wsr[8];
+            float wsr[16];
             v4i Bq[2];
             float asq[2];
             read_b(0, Bq[0], asq[0]);
@@ -380,7 +379,7 @@ __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemmr_kernel(const GemmArgs 
                 __builtin_amdgcn_sched_barrier(0);
             }
         } else {
-            uint32_t wsr[8], wsn[8];
+            float wsr[16];
             v4i Bq[3];
             float asq[3];
             v16i dq[2];
@@ -400,18 +399,17 @@ __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemmr_kernel(const GemmArgs 
                 // a unit after this one that starts a new scale group
                 const bool next_group = u + 1 < 4 && (u + 1) % UPG == 0;
                 if (i + 2 < I) read_b(i + 2, Bq[(i + 2) % 3], asq[(i + 2) % 3]);
-                if (j == 0 && next_group) read_ws((u + 1) / UPG, wsn);
                 if (i + 1 < I) {
                     if ((i + 1) % NT == 0) A = unpack(u + 1);
                     dq[(i + 1) & 1] = mfma32(A, Bq[(i + 1) % 3], zero);
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 chain(j, dq[i & 1], wsr, asq[i % 3]);
-                if (j == NT - 1 && next_group) {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) wsr[e] = wsn[e];
-                }
                 __builtin_amdgcn_sched_barrier(0);
+                // (the next group's scales, once the last chain that uses
+                // this group's has been issued: a second set of 16 registers
+                // would cost the fourth wave per SIMD)
+                if (j == NT - 1 && next_group) read_ws((u + 1) / UPG, wsr);
             }
         }
         st = st == NST - 1 ? 0 : st + 1;
@@ -484,19 +482,27 @@ static int launch_gr(GemmArgs &a, hipStream_t st) {
 }
 
 // Tiles (wave tile 32 rows x 32*NT tokens). The kernel is bound by each
-// SIMD's VALU issue, so what decides is how evenly the 32x32 blocks spread
-// over the SIMDs and how many waves share a SIMD (graph replay, bit-exact,
-// T=2048 K=N=5120 group 32 / T=512 K=17408 N=5120 group 64):
+// SIMD's VALU issue and, nearly as much, by the CU's LDS reads (a wave's
+// scales and operands cost ~37 LDS cycles per 32x32 block and unit against
+// ~33 of VALU per SIMD), so what decides is how evenly the blocks spread over
+// the SIMDs, how many waves share a SIMD and how many token blocks share the
+// scales (graph replay, bit-exact, T=2048 K=N=5120 group 32 / T=512 K=17408
+// N=5120 group 64):
 //   4: 128 x 64, 4 waves of 2 token blocks, four work-groups per CU:
-//     205 / 315 us (the default while its grid gives every CU at least
-//     three work-groups);
-//   9: 128 x 32, 4 waves of one token block, five work-groups per CU:
-//     226 / 277 us (the default for smaller grids);
+//     191 / 264 us (the default while its grid gives every CU at least two
+//     work-groups: N=17408 K=5120 T=300 109 against 129 us for tile 9, N=5120
+//     T=384 with less than one 67 against 59);
+//   9: 128 x 32, 4 waves of one token block: 217 / 234 us (the default for
+//     smaller grids);
 //   0: 160 x 256, 10 waves of 4 token blocks (3, 3, 2, 2 per SIMD), one
-//     work-group per CU: 230 / 760 us;
-//   5: 160 x 64, 10 waves of one token block: 374 / 310 us;
+//     work-group per CU: 187 / 586 us;
+//   5: 160 x 64, 10 waves of one token block: 281 / 221 us;
 //   1, 2, 3, 6, 7, 8: 4- and 5-wave tiles with 4 token blocks, and lean
 //     (one MFMA result live) tiles at 5 or 6 waves per SIMD: all slower.
+// The scales are read as FP32, converted once per stage: a product is then a
+// plain multiplication at twice the rate of v_fma_mix_f32 on FP16 pairs (rate
+// probe, four waves per SIMD: 1.15 against 1.94 ns), 205 -> 194 us; the
+// fourth wave per SIMD (no second set of scale registers) 194 -> 191 us.
 template <int GROUP, bool ZP>
 static int launch_gr_tile(GemmArgs &a, int sel, hipStream_t st) {
     switch (sel) {
@@ -509,7 +515,7 @@ static int launch_gr_tile(GemmArgs &a, int sel, hipStream_t st) {
     case 7: return launch_gr<1, 4, 2, GROUP, ZP, 2, 6>(a, st);    // 128 rows x 64 tokens, 8 waves, lean
     case 8: return launch_gr<2, 4, 1, GROUP, ZP, 2, 5>(a, st);    // 128 rows x 64 tokens, 4 waves, lean
     case 9: return launch_gr<1, 4, 1, GROUP, ZP, 2, 4>(a, st);    // 128 rows x 32 tokens, 4 waves
-    default: return launch_gr<2, 4, 1, GROUP, ZP, 2, 3>(a, st);   // 128 rows x 64 tokens, 4 waves (4)
+    default: return launch_gr<2, 4, 1, GROUP, ZP, 2, 4>(a, st);   // 128 rows x 64 tokens, 4 waves (4)
     }
 }
 
@@ -528,7 +534,7 @@ int launch_gemmr(GemmArgs &a, hipStream_t st) {
         long long tiles = 0;
         for (int i = 0; i < a.count; ++i) tiles += (a.w[i].M / 16 + 7) / 8;
         tiles *= (a.T + 63) / 64;
-        sel = tiles >= 3LL * device_cus() ? 4 : 9;
+        sel = tiles >= 2LL * device_cus() ? 4 : 9;
     }
     const bool zp = a.scale_enc == 1;
     switch (a.group) {
