@@ -37,24 +37,30 @@ from . import _lib
 from ._lib import BF16, F32, SCALE_FP16, SCALE_FP16_ZP4, SCALE_W8, check, lib
 
 
-def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+def _stream() -> int:
+    """The current stream's handle. (The raw-stream getter: building the
+    torch.cuda.Stream object for its handle costs more than the launch.)"""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
-def _ptr(t: Optional[torch.Tensor]):
+def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     if t is None:
         return None
     if not t.is_cuda:
         raise ValueError("tensor must be on the GPU")
     if not t.is_contiguous():
         raise ValueError("tensor must be contiguous")
-    return C.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _need(t, name: str, dtypes, shape, device) -> torch.Tensor:
     """Validate a caller-supplied buffer before its pointer reaches a kernel:
     a tensor on `device` (the weight's GPU), contiguous, of one of `dtypes` and exactly
     `shape`. The kernels trust these sizes, so a mismatch raises here."""
+    # a buffer as it should be passes one test; the checks below only name what is wrong
+    if (isinstance(t, torch.Tensor) and t.shape == shape and t.device == device and t.is_contiguous()
+            and (t.dtype is dtypes or (dtypes.__class__ is tuple and t.dtype in dtypes))):
+        return t
     if not isinstance(t, torch.Tensor):
         raise ValueError(f"{name} must be a torch.Tensor")
     if t.device != torch.device(device):
@@ -73,12 +79,14 @@ def _need(t, name: str, dtypes, shape, device) -> torch.Tensor:
 _BITS16 = (torch.int16, torch.uint16) if hasattr(torch, "uint16") else (torch.int16,)
 
 
+_DTYPE_CODES = {torch.float32: F32, torch.bfloat16: BF16}
+
+
 def _dtype_code(dt: torch.dtype) -> int:
-    if dt == torch.float32:
-        return F32
-    if dt == torch.bfloat16:
-        return BF16
-    raise ValueError(f"unsupported dtype {dt}")
+    code = _DTYPE_CODES.get(dt)
+    if code is None:
+        raise ValueError(f"unsupported dtype {dt}")
+    return code
 
 
 @dataclass
@@ -318,7 +326,7 @@ def _residual(residual, T: int, M: int, device):
 
 
 def _check_weight(w: "W4Weight", device):
-    if not torch.device(device).type == "cuda":
+    if (device if isinstance(device, torch.device) else torch.device(device)).type != "cuda":
         raise ValueError("weights must be on the GPU")
     nbytes = w.M * w.K if w.scale_enc == SCALE_W8 else w.M * w.K // 2
     _need(w.codes, "weight codes", torch.uint8, (nbytes,), device)
