@@ -36,19 +36,22 @@ constexpr int kW4GroupTT = 4;      // token tiles per raster group
 
 #define KXW4_W4_LDS(p) ((__attribute__((address_space(3))) void *)(p))
 
-// Four int8 bytes w - zp from four nibbles held as w + 8 (the packed dword
-// XOR 0x88888888, masked to one nibble per byte); c = (120 - zp) * 0x01010101.
-// The byte sums w + 128 - zp stay in [113, 143], so no carry crosses a byte,
-// and the XOR turns the excess-128 bytes into two's complement.
-__device__ __forceinline__ uint32_t zp_bytes(uint32_t u, uint32_t c) { return (u + c) ^ 0x80808080u; }
+// Four int8 bytes w - zp from the low nibbles n (two's complement w) of u's
+// bytes: one three-input bit operation makes each byte 0x80 | (n ^ 8) =
+// 128 + w + 8; subtracting zz = (zp + 8) * 0x01010101 leaves 128 + w - zp in
+// [113, 143] per byte, so no borrow crosses a byte, and the XOR turns the
+// excess-128 bytes into two's complement.
+__device__ __forceinline__ uint32_t zp_bytes(uint32_t u, uint32_t zz) {
+    const uint32_t e = ((u ^ 0x08080808u) & 0x0F0F0F0Fu) | 0x80808080u;
+    return (e - zz) ^ 0x80808080u;
+}
 
-__device__ __forceinline__ v4i unpack_k64_zp(uint32_t d0, uint32_t d1, uint32_t c) {
-    const uint32_t x0 = d0 ^ 0x88888888u, x1 = d1 ^ 0x88888888u;
+__device__ __forceinline__ v4i unpack_k64_zp(uint32_t d0, uint32_t d1, uint32_t zz) {
     v4i b;
-    b.x = (int)zp_bytes(x0 & 0x0F0F0F0Fu, c);
-    b.y = (int)zp_bytes((x0 >> 4) & 0x0F0F0F0Fu, c);
-    b.z = (int)zp_bytes(x1 & 0x0F0F0F0Fu, c);
-    b.w = (int)zp_bytes((x1 >> 4) & 0x0F0F0F0Fu, c);
+    b.x = (int)zp_bytes(d0, zz);
+    b.y = (int)zp_bytes(d0 >> 4, zz);
+    b.z = (int)zp_bytes(d1, zz);
+    b.w = (int)zp_bytes(d1 >> 4, zz);
     return b;
 }
 
@@ -228,7 +231,7 @@ __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void w4a4_kernel(const W4a4Args a
             for (int u = 0; u < UPS; ++u) {
                 const uint32_t p = *reinterpret_cast<const uint16_t *>(sb + soff_lds + (jb * 2 * UPS + u) * 32);
                 w[jb][u] = half_bits_to_float((uint16_t)(p & 0xFFF0u));
-                zc[u] = (uint32_t)(120 - sext4(p)) * 0x01010101u;
+                zc[u] = (uint32_t)(sext4(p) + 8) * 0x01010101u;
             }
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -407,23 +410,29 @@ static int launch_w4(W4a4Args &a, hipStream_t st) {
 }
 
 int launch_w4a4(W4a4Args &a, hipStream_t st) {
-    // Default 128 x 64 (three work-groups per CU); when that grid gives fewer
-    // than two work-groups per CU, 64 x 64 (twice the work-groups, more waves
-    // per SIMD to overlap one wave's chain with another's MFMAs: cfg2 M=512
-    // 196 -> 184 us). The 64 x 160 tile (10 waves, one work-group per CU)
-    // balances the cfg2 M=512 grid but measures slower (207 us): with one
-    // token block per wave the zero-point weight unpack is no longer shared.
+    // 64 x 64 or 128 x 64, whichever loads the busiest CU less. At
+    // K = 17408 a 64 x 64 tile takes a CU 46-51 us and a 128 x 64 tile, whose
+    // two token blocks share the weight unpack, 88-95 us: 1.87 times as long
+    // for twice the work, so the smaller tile wins where its finer grid
+    // saves more than that. N = 5120, K = 17408, 64 x 64 against 128 x 64: T = 64
+    // 98 against 134 us, T = 512 154.7 / 179.8, T = 1024 252 / 284, T = 2048
+    // 463 / 441; N = 17408, K = 5120, T = 512 128.5 / 134.2. (128 x 64 at two
+    // or more work-groups per CU, as before, gave 171 us at T = 512 cold and
+    // 302 at T = 1024; 64 x 160 with 10 waves 197 at T = 512, since with one
+    // token block per wave the zero-point weight unpack is not shared.)
     // the w4a4_tile option (0..4) picks one configuration (tests, tuning)
     int sel = options().w4a4_tile;
     if (sel < 0) {
-        const long long tiles = (long long)((a.T + 127) / 128) * ((a.M / 16 + 3) / 4);
-        sel = tiles < 2LL * device_cus() ? 4 : 0;
+        const long long cus = device_cus(), nt = (a.M / 16 + 3) / 4;
+        const long long big = (((a.T + 127) / 128) * nt + cus - 1) / cus;
+        const long long small = (((a.T + 63) / 64) * nt + cus - 1) / cus;
+        sel = 100 * small < 187 * big ? 4 : 0;
     }
     switch (sel) {
     case 3: return launch_w4<1, 1, 2, 5, 3, 3>(a, st);      // 64 tokens x 160 rows, 10 waves
     case 1: return launch_w4<2, 1, 2, 4, 3, 2>(a, st);      // 128 tokens x 128 rows, 8 waves
     case 2: return launch_w4<1, 2, 2, 2, 3, 2>(a, st);      // 64 tokens x 128 rows, 4 waves
-    case 4: return launch_w4<1, 1, 2, 2, 3, 3>(a, st);      // 64 tokens x 64 rows, 4 waves
+    case 4: return launch_w4<1, 1, 2, 2, 3, 4>(a, st);      // 64 tokens x 64 rows, 4 waves
     default: return launch_w4<2, 1, 2, 2, 3, 2>(a, st);     // 128 tokens x 64 rows, 4 waves
     }
 }
