@@ -351,22 +351,50 @@ int device_cus() {
     return cus[dev];
 }
 
+// Launches that the row-wave kernel runs faster than the strip kernel; it cuts
+// the rows evenly over the CUs and stages the activations once per
+// work-group. (rgs: row-groups; measured with 600 MB of weights in turn, so
+// that they come from HBM, strip against row-wave kernel.)
+static bool rowwave_first(const DecodeArgs &a, int rgs) {
+    const int cus = device_cus();
+    if (a.w8) {
+        // full rounds of two work-groups of 16 row-groups per CU, one split
+        // and long rows (248,320 rows, K = 5120: T = 1 234.6 against 230.9
+        // us, T = 8 237.8-239 both ways; K = 8192: T = 1 374 against 353);
+        // rounds that are not full lose (200,000 rows, K = 5120, T = 1: 184
+        // against 205), and so do shorter rows (248,320 rows, K = 4096: 179
+        // against 186)
+        const int per = 16 * cus, wgs = (rgs + per - 1) / per;
+        return a.T <= 8 && a.K >= 4608 && a.w[0].seg_split[0] == 1 && wgs % 2 == 0 && 10ll * rgs >= 9ll * wgs * per;
+    }
+    if (a.block != 0) return false;
+    // many rows (8 tokens, K = 5120, 34,816 rows: 20.9 against 18.5 us)
+    if (a.T > 2 && rgs > 6 * cus) return true;
+    // a GEMM of two row-groups per CU or more (N = 17408, K = 5120: T = 4
+    // 14.1 against 11.4 us, T = 13 16.1 against 13.6; N = 8192: T = 8 9.4
+    // against 8.5), but few tokens at short rows of few row-groups (N = 14336,
+    // K = 2048, T = 4: 7.6 against 8.0)
+    if (a.variant == kVarGemm)
+        return a.T > 2 && rgs >= 2 * cus && (a.T > 4 || rgs > 4 * cus || a.K >= 8192);
+    // a GEMV of few rows that are long (N = 2048, K = 12288, T = 1: 8.1
+    // against 6.6 us; N = 5120, K = 17408, group 64: 13.1 against 12.1; at
+    // N = 3072, K = 5120 both take 6.0)
+    return a.T <= 4 && rgs <= 2 * cus && a.K > 8192;
+}
+
 int launch_decode(DecodeArgs &a, bool debug, hipStream_t st) {
-    // Every mode the strip kernel takes goes there, but for one: per-token
-    // launches of 3-16 tokens over many rows stay on the row-wave kernel,
-    // which cuts the rows evenly over the CUs and stages the activations
-    // once per work-group (8 tokens, K = 5120, 34,816 rows: 18.5 against
-    // 20.9 us; 17,408 rows: 12.4 against 11.3 us). The decode_kernel option
-    // forces the K-parallel kernel below (kparallel) or prefers the row-wave
-    // kernel (rowwave, as a rowwave_* option does); the modes the strip
-    // kernel is not built for (per-token activations with zero points or
-    // group 32, K32 blocks with plain FP16 scales) run on those two.
+    // Every mode the strip kernel takes goes there, but for the launches of
+    // rowwave_first. The decode_kernel option forces the K-parallel kernel
+    // below (kparallel) or prefers the row-wave kernel (rowwave, as a
+    // rowwave_* option does); the modes the strip kernel is not built for
+    // (per-token activations with zero points or group 32, K32 blocks with
+    // plain FP16 scales) run on those two.
     const int force = options().decode_kernel;
     const bool rw_opt = options().rowwave_spw || options().rowwave_ring || options().rowwave_k;
     if (!debug && force == kDecodeAuto && !rw_opt && strip_takes(a.group, a.block, a.scale_enc, a.T, a.K)) {
         int rgs = 0;
         for (int i = 0; i < a.count; ++i) rgs += a.w[i].M / 16;
-        if (a.block == 0 && a.T > 2 && a.T <= 16 && rgs > 6 * device_cus()) {
+        if (a.T <= 16 && rowwave_first(a, rgs)) {
             const int r = launch_rowwave(a, st);
             if (r != 1) return r;
         }

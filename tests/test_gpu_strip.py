@@ -112,3 +112,30 @@ def test_strip_packed_segments(mode, rows, segs):
     for (c, s, _), y in zip(ws, ys):
         sp = O.segment_splits(T, c.shape[0], K, off)
         check(y, oracle(mode, c, s, act, O.VAR_GEMM, sp), f"{mode} rows={c.shape[0]}")
+
+
+# either side of the lines between the strip and the row-wave kernel: the first
+# and last rows against the oracle, with the whole weight's split plan
+@pytest.mark.parametrize("mode,call,T,M,K", [
+    ("token64", "gemm", 5, 8192, 256), ("token64", "gemm", 5, 8176, 256), ("token128", "gemm", 4, 16400, 256),
+    ("token128", "gemm", 4, 16384, 256), ("token128", "gemm", 3, 8192, 8192), ("token128", "gemm", 2, 16400, 256),
+    ("token64", "gemm", 16, 8208, 12288),
+    ("token64", "gemv", 4, 48, 8320), ("token64", "gemv", 5, 48, 8320), ("token128", "gemv", 1, 48, 8192),
+    ("token128", "gemv", 2, 8192, 8320), ("token128", "gemv", 1, 8208, 8320),
+    ("w8", "gemm", 8, 117984, 4608), ("w8", "gemm", 9, 117984, 4608), ("w8", "gemv", 1, 131072, 4608)])
+def test_strip_rowwave_line(mode, call, T, M, K):
+    group, block, enc = MODES[mode]
+    g = torch.Generator(device=DEV).manual_seed(T * M + K)
+    lim = (-128, 128) if mode == "w8" else (-8, 8)
+    codes = torch.randint(*lim, (M, K), generator=g, device=DEV, dtype=torch.int8)
+    bits = (0.02 * torch.rand(M, K // group, generator=g, device=DEV)).to(torch.float16).view(torch.int16)
+    w = ops.W4Weight.from_codes_s8(codes, bits) if mode == "w8" else ops.W4Weight.from_codes(codes, bits, group, enc)
+    x = torch.randn(T, K, generator=g, device=DEV).cpu().numpy()
+    a, act = ops.quantize_act(dev(x), block), O.quantize_act(x, block)
+    if call == "gemm":
+        y, var, sp = ops.gemm(w, a), O.VAR_GEMM, O.segment_splits(T, M, K)
+    else:
+        y, var, sp = ops.gemv(w, a), O.VAR_GEMV, O.gemv_splits(M // 16)
+    for lo in (0, M - 48):
+        c, s = codes[lo:lo + 48].cpu().numpy(), bits[lo:lo + 48].cpu().numpy().view(np.uint16)
+        check(y[:, lo:lo + 48].contiguous(), oracle(mode, c, s, act, var, sp), f"{mode} {call} T={T} M={M} K={K} row {lo}")
