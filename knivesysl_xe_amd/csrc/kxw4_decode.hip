@@ -391,19 +391,28 @@ int launch_decode(DecodeArgs &a, bool debug, hipStream_t st) {
     // plain FP16 scales) run on those two.
     const int force = options().decode_kernel;
     const bool rw_opt = options().rowwave_spw || options().rowwave_ring || options().rowwave_k;
-    if (!debug && force == kDecodeAuto && !rw_opt && strip_takes(a.group, a.block, a.scale_enc, a.T, a.K)) {
+    const bool strip_ok = !debug && strip_takes(a.group, a.block, a.scale_enc, a.T, a.K);
+    auto strip = [&]() {
+        StripArgs s = strip_args(a, a.variant, 1, 16);
+        return launch_strip(s, st);
+    };
+    if (strip_ok && force == kDecodeAuto && !rw_opt) {
         int rgs = 0;
         for (int i = 0; i < a.count; ++i) rgs += a.w[i].M / 16;
         if (a.T <= 16 && rowwave_first(a, rgs)) {
             const int r = launch_rowwave(a, st);
             if (r != 1) return r;
         }
-        StripArgs s = strip_args(a, a.variant, 1, 16);
-        return launch_strip(s, st);
+        return strip();
     }
-    // W8 and K16 weights have no K-parallel instance; 1 hands the shape
-    // back to the caller (the GEMM path for W8)
-    if (a.w8 || a.group == 16) return debug ? 1 : launch_rowwave(a, st);
+    // W8 and K16 weights have no K-parallel instance: what the row-wave
+    // kernel hands back (long K, whose activations do not fit its LDS) runs on
+    // the strip kernel; 1 hands the debug partials back to the caller (the
+    // GEMM path for W8)
+    if (a.w8 || a.group == 16) {
+        const int r = debug ? 1 : launch_rowwave(a, st);
+        return r == 1 && strip_ok ? strip() : r;
+    }
     bool no_rowwave = force == kDecodeKParallel;
     if (force == kDecodeAuto && a.block == 0 && a.scale_enc == 0 && a.T <= 8) {
         // per-token group 32 with at most one row-group per CU: one

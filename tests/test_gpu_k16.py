@@ -75,9 +75,7 @@ def test_k16_gemv(M, K, T, splits):
 
 @pytest.mark.parametrize("M,T", [(1040, 8), (1040, 16), (5120, 16), (5120, 1), (5120, 2)])
 def test_k16_gemv_long_k(M, T):
-    # K = 17408 (the down projection): T tokens' activations do not fit in one
-    # work-group's LDS with the scale tables, so the launcher runs the tokens
-    # in chunks that do; the last chunk is shorter
+    # K = 17408 (the down projection): the strip kernel streams any K
     K = 17408
     print(f"k16 gemv long K M={M} K={K} T={T}", flush=True)
     rng = np.random.default_rng(620 + T + M)

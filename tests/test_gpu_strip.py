@@ -1,6 +1,8 @@
 """The strip kernel (csrc/kxw4_strip.hip) at the edges of its tiles, stages
 and split plans, against the oracle: int32 partials and the order of every
 FP32 step are fixed, so the outputs must be the oracle's bits."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -139,3 +141,32 @@ def test_strip_rowwave_line(mode, call, T, M, K):
     for lo in (0, M - 48):
         c, s = codes[lo:lo + 48].cpu().numpy(), bits[lo:lo + 48].cpu().numpy().view(np.uint16)
         check(y[:, lo:lo + 48].contiguous(), oracle(mode, c, s, act, var, sp), f"{mode} {call} T={T} M={M} K={K} row {lo}")
+
+
+def launches(call):
+    """Kernel launches of `call`, counted as the nodes of its captured graph."""
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        call()
+    n = C.c_size_t()
+    assert C.CDLL(path).hipGraphGetNodes(C.c_void_p(g.raw_cuda_graph()), None, C.byref(n)) == 0
+    return n.value
+
+
+# long K at 8 and 16 tokens: the row-wave kernel's LDS does not hold the
+# activations, and one launch that reads the weight once takes all of them
+@pytest.mark.parametrize("mode,T", [("w8", 8), ("w8", 16), ("k16", 8), ("k16", 16)])
+def test_long_k_reads_the_weight_once(mode, T):
+    rng = np.random.default_rng(900 + T)
+    M, K = 80, 17408
+    codes, scales, w = weight(rng, mode, M, K)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    a, act = ops.quantize_act(dev(x), 32), O.quantize_act(x, 32)
+    want = oracle(mode, codes, scales, act, O.VAR_GEMV, O.gemv_splits(M // 16))
+    for option in (0, 2):                                # the default dispatch, the row-wave kernel preferred
+        with ops.option("decode_kernel", option):
+            y = ops.gemv(w, a)
+            check(y, want, f"{mode} T={T}")
+            assert launches(lambda: ops.gemv(w, a, out=y)) == 1
