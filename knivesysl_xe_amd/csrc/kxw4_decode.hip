@@ -29,6 +29,7 @@
 // partials need.
 #include "kxw4_device.hpp"
 #include "kxw4_internal.hpp"
+#include "kxw4_route.hpp"
 
 #include <algorithm>
 
@@ -46,13 +47,6 @@ struct DcStage {
     v4u wd;
     v4i A[AT == 0 ? 1 : 2 * AT];
 };
-
-// LDS words: partials [nu][tl][16] int32, scales [g][16] uint16, split
-// partials [smax][tl][16] float, in the general mode the activation scale and
-// code sum [nu][tl], then 64 dummy words.
-__host__ __device__ inline int decode_lds_words(int nu, int g, int tl, int smax, bool side) {
-    return nu * tl * 16 + g * 8 + smax * tl * 16 + (side ? 2 * nu * tl : 0) + 64;
-}
 
 template <int AT, int UNIT, int MODE, bool DEBUG, int PFW>
 __global__ __launch_bounds__(kDcThreads) void decode_kernel(const DecodeArgs a) {
@@ -351,44 +345,24 @@ int device_cus() {
     return cus[dev];
 }
 
-// Launches that the row-wave kernel runs faster than the strip kernel; it cuts
-// the rows evenly over the CUs and stages the activations once per
-// work-group. (rgs: row-groups; measured with 600 MB of weights in turn, so
-// that they come from HBM, strip against row-wave kernel.)
-static bool rowwave_first(const DecodeArgs &a, int rgs) {
-    const int cus = device_cus();
-    if (a.w8) {
-        // full rounds of two work-groups of 16 row-groups per CU, one split
-        // and long rows (248,320 rows, K = 5120: T = 1 234.6 against 230.9
-        // us, T = 8 237.8-239 both ways; K = 8192: T = 1 374 against 353);
-        // rounds that are not full lose (200,000 rows, K = 5120, T = 1: 184
-        // against 205), and so do shorter rows (248,320 rows, K = 4096: 179
-        // against 186)
-        const int per = 16 * cus, wgs = (rgs + per - 1) / per;
-        return a.T <= 8 && a.K >= 4608 && a.w[0].seg_split[0] == 1 && wgs % 2 == 0 && 10ll * rgs >= 9ll * wgs * per;
+// The launch as the dispatch rule sees it.
+static DecodeShape decode_shape(const DecodeArgs &a) {
+    DecodeShape s{device_cus(), 0, a.T, a.K, a.group, a.w[0].seg_split[0], a.block != 0, a.w8 != 0};
+    for (int i = 0; i < a.count; ++i) {
+        s.rgs += a.w[i].M / 16;
+        for (int g = 0; g < a.seg_count; ++g)
+            if (a.w[i].seg_split[g] != a.w[0].seg_split[0]) s.S = 0;
     }
-    if (a.block != 0) return false;
-    // many rows (8 tokens, K = 5120, 34,816 rows: 20.9 against 18.5 us)
-    if (a.T > 2 && rgs > 6 * cus) return true;
-    // a GEMM of two row-groups per CU or more (N = 17408, K = 5120: T = 4
-    // 14.1 against 11.4 us, T = 13 16.1 against 13.6; N = 8192: T = 8 9.4
-    // against 8.5), but few tokens at short rows of few row-groups (N = 14336,
-    // K = 2048, T = 4: 7.6 against 8.0)
-    if (a.variant == kVarGemm)
-        return a.T > 2 && rgs >= 2 * cus && (a.T > 4 || rgs > 4 * cus || a.K >= 8192);
-    // a GEMV of few rows that are long (N = 2048, K = 12288, T = 1: 8.1
-    // against 6.6 us; N = 5120, K = 17408, group 64: 13.1 against 12.1; at
-    // N = 3072, K = 5120 both take 6.0)
-    return a.T <= 4 && rgs <= 2 * cus && a.K > 8192;
+    return s;
 }
 
 int launch_decode(DecodeArgs &a, bool debug, hipStream_t st) {
-    // Every mode the strip kernel takes goes there, but for the launches of
-    // rowwave_first. The decode_kernel option forces the K-parallel kernel
-    // below (kparallel) or prefers the row-wave kernel (rowwave, as a
-    // rowwave_* option does); the modes the strip kernel is not built for
-    // (per-token activations with zero points or group 32, K32 blocks with
-    // plain FP16 scales) run on those two.
+    // The modes the strip kernel is built for go where decode_route says. The
+    // decode_kernel option forces the K-parallel kernel below (kparallel) or
+    // prefers the row-wave kernel (rowwave, as a rowwave_* option does); the
+    // modes the strip kernel is not built for (per-token activations with
+    // zero points or group 32, K32 blocks with plain FP16 scales) run on those
+    // two.
     const int force = options().decode_kernel;
     const bool rw_opt = options().rowwave_spw || options().rowwave_ring || options().rowwave_k;
     const bool strip_ok = !debug && strip_takes(a.group, a.block, a.scale_enc, a.T, a.K);
@@ -396,14 +370,16 @@ int launch_decode(DecodeArgs &a, bool debug, hipStream_t st) {
         StripArgs s = strip_args(a, a.variant, 1, 16);
         return launch_strip(s, st);
     };
-    if (strip_ok && force == kDecodeAuto && !rw_opt) {
-        int rgs = 0;
-        for (int i = 0; i < a.count; ++i) rgs += a.w[i].M / 16;
-        if (a.T <= 16 && rowwave_first(a, rgs)) {
+    const bool routed = strip_ok && force == kDecodeAuto && !rw_opt;
+    bool no_rowwave = force == kDecodeKParallel;
+    if (routed) {
+        const DecodeRoute route = decode_route(decode_shape(a));
+        if (route == kRouteRowwave) {
             const int r = launch_rowwave(a, st);
             if (r != 1) return r;
         }
-        return strip();
+        if (route != kRouteKParallel) return strip();
+        no_rowwave = true;
     }
     // W8 and K16 weights have no K-parallel instance: what the row-wave
     // kernel hands back (long K, whose activations do not fit its LDS) runs on
@@ -413,8 +389,7 @@ int launch_decode(DecodeArgs &a, bool debug, hipStream_t st) {
         const int r = debug ? 1 : launch_rowwave(a, st);
         return r == 1 && strip_ok ? strip() : r;
     }
-    bool no_rowwave = force == kDecodeKParallel;
-    if (force == kDecodeAuto && a.block == 0 && a.scale_enc == 0 && a.T <= 8) {
+    if (!no_rowwave && force == kDecodeAuto && a.block == 0 && a.scale_enc == 0 && a.T <= 8) {
         // per-token group 32 with at most one row-group per CU: one
         // work-group per row-group whose waves read consecutive kilobytes
         // beats the row-wave kernel's per-split streams, except for one or
@@ -428,21 +403,18 @@ int launch_decode(DecodeArgs &a, bool debug, hipStream_t st) {
         const int r = launch_rowwave(a, st);
         if (r != 1) return r;
     }
-    constexpr size_t kBudget = 64 * 1024;
     const int unit = a.block == 32 ? 32 : a.group;
     const int nu = a.K / unit, g = a.K / a.group;
-    if (2 * g > kScaleChunks * kDcThreads) return -2;
+    // (a K that one row-group's partials or scales do not fit the LDS for)
+    if (2 * g > kScaleChunks * kDcThreads) return routed ? strip() : -2;
     const int mode = (a.block == 0 && a.scale_enc == 0) ? 0 : 1;
     const bool side = mode != 0 || debug;
     int smax = 1;
     for (int i = 0; i < a.count; ++i)
         for (int s = 0; s < a.seg_count; ++s) smax = std::max(smax, a.w[i].seg_split[s]);
     a.smax = smax;
-    // token slice: the largest (at most 64) whose partials fit in LDS
-    auto bytes = [&](int ts) { return (size_t)4 * decode_lds_words(nu, g, ts, smax, side); };
-    int ts = a.T < 64 ? a.T : 64;
-    while (ts > 1 && bytes(ts) > kBudget) ts = (ts + 1) / 2;
-    if (bytes(ts) > kBudget) return -2;
+    const int ts = kparallel_slice(nu, g, a.T, smax, side);
+    if (ts == 0) return routed ? strip() : -2;
     a.ts = ts;
     int rgs = 0;
     for (int i = 0; i < a.count; ++i) {
@@ -451,7 +423,7 @@ int launch_decode(DecodeArgs &a, bool debug, hipStream_t st) {
     }
     a.total_rg = rgs;
     const dim3 grid(rgs, (a.T + ts - 1) / ts);
-    const size_t lds = bytes(ts);
+    const size_t lds = (size_t)4 * decode_lds_words(nu, g, ts, smax, side);
     if (ts <= 8) return launch_dc_unit<0>(a, unit, mode, debug, grid, lds, st);
     if (ts <= 16) return launch_dc_unit<1>(a, unit, mode, debug, grid, lds, st);
     if (ts <= 32) return launch_dc_unit<2>(a, unit, mode, debug, grid, lds, st);

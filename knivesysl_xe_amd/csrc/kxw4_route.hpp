@@ -1,0 +1,126 @@
+// kxw4_route.hpp — which kernel a decode launch (at most 16 tokens) runs on:
+// the strip kernel (kxw4_strip.hip), the row-wave kernel (kxw4_rowwave.hip)
+// or the K-parallel kernel (kxw4_decode.hip). Plain C++, so that the rule can
+// be checked without a GPU.
+//
+// Every kernel gives the same bits; the lines lie where the times cross. They
+// were measured over 256-73,728 rows (W8: 262,144) of 1,024-17,408 columns
+// and 1-16 tokens, launches of a graph replay over 620 MB of weights in turn,
+// so that the weights come from HBM (figures: us a launch, MI355X, 256 CUs).
+// A shape that the row-wave kernel has no LDS for goes on to the strip kernel.
+#pragma once
+
+namespace kxw4 {
+
+enum DecodeRoute { kRouteStrip = 0, kRouteRowwave = 1, kRouteKParallel = 2 };
+
+struct DecodeShape {
+    int cus;                          // compute units of the device
+    int rgs;                          // 16-row groups over all weights
+    int T, K, group;
+    int S;                            // split count of every token and weight, 0 if they differ
+    bool blocks;                      // activation scales per K32 block, else per token
+    bool w8;
+};
+
+// The K-parallel kernel's LDS words for slices of `tl` tokens: partials
+// [nu][tl][16] int32, scales [g][16] uint16, split partials [smax][tl][16]
+// float, in the general mode the activation scale and code sum [nu][tl], then
+// 64 dummy words.
+constexpr int decode_lds_words(int nu, int g, int tl, int smax, bool side) {
+    return nu * tl * 16 + g * 8 + smax * tl * 16 + (side ? 2 * nu * tl : 0) + 64;
+}
+
+// Its tokens per slice: the most (at most 64) whose LDS fits in 64 KB, 0 if
+// one token's does not.
+inline int kparallel_slice(int nu, int g, int T, int smax, bool side) {
+    int ts = T < 64 ? T : 64;
+    while (ts > 1 && 4ll * decode_lds_words(nu, g, ts, smax, side) > 64 * 1024) ts = (ts + 1) / 2;
+    return 4ll * decode_lds_words(nu, g, ts, smax, side) > 64 * 1024 ? 0 : ts;
+}
+
+// W8: a row-wave work-group takes 16 row-groups, so the rows are good for it
+// where they fill the CUs and are long: from four rounds on (245,760 rows, K
+// = 5120: strip 240 against 235 us at T = 8; 248,320: 239 / 233; 393,216: 381
+// / 372; rounds that are 15/16 full or more: 294,912 rows take 291 / 292),
+// from two at K = 8192 (122,880 rows, T = 4: 196 / 187), and in one round past
+// eight tokens (57,344 rows, K = 5120, T = 12: 67 / 60; 65,536: 76 / 71). Two
+// and three rounds of shorter rows tie, emptier ones lose (200,000 rows, T =
+// 1: 189 / 210), still shorter rows too (65,536 rows, K = 4096, T = 8: 54 /
+// 61).
+inline DecodeRoute route_w8(const DecodeShape &s) {
+    if (s.S != 1 || s.K < 4608) return kRouteStrip;
+    const long long per = 16ll * s.cus, rounds = (s.rgs + per - 1) / per;
+    if (rounds >= 4 || (rounds >= 2 && s.K >= 8192))
+        return 16ll * s.rgs >= 15 * rounds * per ? kRouteRowwave : kRouteStrip;
+    return rounds == 1 && s.T > 8 && 8ll * s.rgs >= 7 * per ? kRouteRowwave : kRouteStrip;
+}
+
+// Reference mode: many rows in one split, group 64 (34,816 rows, K = 5120, T
+// = 4: 32.4 / 29.8; 65,536 rows, T = 8: 45.9 / 43.0; at group 32 both take the
+// same), and two splits where the rows fill six row-groups per CU and no more
+// (24,576 rows, K = 8192, T = 4: 31.9 / 28.6 at group 64, 32.4 / 30.3 at 32;
+// 26,624 rows tie or lose). One or two tokens stay on the strips, whose
+// chains run on the real tokens alone.
+inline DecodeRoute route_blocks(const DecodeShape &s) {
+    if (s.T <= 2 || s.group == 16) return kRouteStrip;
+    if (s.S == 1) return s.group == 64 && s.rgs >= 8 * s.cus ? kRouteRowwave : kRouteStrip;
+    return s.S == 2 && s.K >= 4096 && s.rgs > 5 * s.cus && s.rgs <= 6 * s.cus ? kRouteRowwave : kRouteStrip;
+}
+
+// Per token. The row-wave kernel cuts the rows evenly over the CUs and keeps
+// four tiles of weights in flight per wave, which long streams reward; the
+// strips run more splits of more rows side by side.
+inline DecodeRoute route_token(const DecodeShape &s) {
+    const int T = s.T, K = s.K, cus = s.cus;
+    const bool g64 = s.group == 64;
+    auto rowwave = [](bool yes) { return yes ? kRouteRowwave : kRouteStrip; };
+    // one or two splits: enough rows to stream (34,816 rows, K = 5120, T = 1:
+    // strip 22.6 against row-wave 18.4 us; 17,408 rows, T = 2 14.6 / 11.6, T =
+    // 16 16.6 / 14.5). (Short rows in two splits of one or two tokens at
+    // group 128: 28,480 rows, K = 2432 9.7 / 10.8.)
+    if (s.S <= 2) return rowwave(!(s.S == 2 && T <= 2 && !g64 && K < 2560 && s.rgs > 5 * cus));
+    if (s.rgs <= cus) {
+        // At most one row-group per CU: the K-parallel kernel reads a
+        // row-group in consecutive kilobytes by one work-group. It is ahead
+        // while its token slices are short (past five tokens the chains of a
+        // slice take over: 640 rows, K = 6144, T = 8, one slice of eight:
+        // strip 7.7 against 9.2 us; K = 7936, two of four: 9.0 / 7.5) and all
+        // resident at once (3,072 rows, K = 17408, T = 4: 12.4 / 15.9).
+        // Sixteen splits (the GEMM plan): 1,024 rows, group 128, K = 12288, T =
+        // 1 8.5 / 6.8; K = 17408, T = 16 12.6 / 10.3; group 64, K = 3840, T = 1
+        // 6.4 / 5.4.
+        const int nu = K / s.group, ts = kparallel_slice(nu, nu, T, s.S, false);
+        const bool kpar = ts > 0 && ts <= 5 && (long long)s.rgs * ((T + ts - 1) / ts) <= cus;
+        if (s.S == 16) return kpar && K > (T <= 4 ? 1024 : 2048) ? kRouteKParallel : kRouteStrip;
+        if (s.S != 8 || T > 4) return kRouteStrip;
+        // eight splits (the GEMV plan): 2,048 rows, K = 8192, group 64, T = 1
+        // strip 6.8 against row-wave 5.6 us; K = 17408, T = 3 10.9 / 10.0;
+        // group 128, K = 12288, T = 4 8.7 / K-parallel 8.0
+        if (T <= 2) return rowwave(K > (g64 ? 2048 : 4096));
+        if (g64) return rowwave(K > 8192);
+        return kpar && K > 4096 ? kRouteKParallel : kRouteStrip;
+    }
+    // More rows, four splits and up.
+    const bool two = s.rgs <= 2 * cus;
+    const int kmin = g64 ? 6144 : 8192;
+    // 8,192 rows in four splits, group 64: K = 4096, T = 1 7.6 / 6.8 us; 6,144
+    // rows in eight: K = 8192, T = 2 9.0 / 8.4
+    if (T <= 2) return rowwave(s.S == 4 ? K >= (two ? 4096 : 6144) : two && K >= kmin);
+    // 14,336 rows in four splits, K = 8192, T = 8: 17.4 / 15.3; 6,144 rows in
+    // eight, group 64, K = 12288: 14.6 / 12.6 (17,408 rows in eight, K = 5120,
+    // T = 4: 19.5 / 27.8)
+    if (T <= 8) return rowwave(s.S == 4 ? K >= 6144 : T > 4 && two && K >= kmin);
+    // 6,144 rows, K = 12288, T = 12: 15.6 / 13.3; 16,384 rows in eight, K =
+    // 8192: 25.6 / 21.4 (10,240 rows: 15.2 / 19.5)
+    return rowwave(K >= (g64 ? 4608 : 6144) && (two || (s.rgs > 3 * cus && s.rgs <= 4 * cus)));
+}
+
+// The launch's kernel among those built for its mode (strip_takes).
+inline DecodeRoute decode_route(const DecodeShape &s) {
+    if (s.T > 16 || s.S == 0) return kRouteStrip;
+    if (s.w8) return route_w8(s);
+    return s.blocks ? route_blocks(s) : route_token(s);
+}
+
+}  // namespace kxw4

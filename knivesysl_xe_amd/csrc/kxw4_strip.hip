@@ -33,7 +33,7 @@
 // (GEMV, group 64), T = 16 371 -> 22 us, T = 64 4477 -> 70 us; fan-out over
 // 34,816 rows, K = 5120, T = 1 64 -> 23.4 us; per-token N = 5120, K = 17408,
 // T = 64 118 -> 33 us (some per-token and W8 launches of up to 16 tokens stay
-// on the row-wave kernel: rowwave_first in kxw4_decode.hip); K16 N = 5120, K = 17408: T = 1
+// on the row-wave kernel: kxw4_route.hpp); K16 N = 5120, K = 17408: T = 1
 // 36 -> 19.2 us, T = 16 323 -> 30 us; W8 N = 17408, K = 5120: T = 8 30 -> 22
 // us, T = 64 140 -> 43 us, T = 256 401 -> 119 us.
 #include "kxw4_device.hpp"

@@ -116,15 +116,27 @@ def test_strip_packed_segments(mode, rows, segs):
         check(y, oracle(mode, c, s, act, O.VAR_GEMM, sp), f"{mode} rows={c.shape[0]}")
 
 
-# either side of the lines between the strip and the row-wave kernel: the first
-# and last rows against the oracle, with the whole weight's split plan
+# either side of the lines between the strip, the row-wave and the K-parallel
+# kernel (csrc/kxw4_route.hpp): the first and last rows against the oracle,
+# with the whole weight's split plan
 @pytest.mark.parametrize("mode,call,T,M,K", [
     ("token64", "gemm", 5, 8192, 256), ("token64", "gemm", 5, 8176, 256), ("token128", "gemm", 4, 16400, 256),
     ("token128", "gemm", 4, 16384, 256), ("token128", "gemm", 3, 8192, 8192), ("token128", "gemm", 2, 16400, 256),
     ("token64", "gemm", 16, 8208, 12288),
     ("token64", "gemv", 4, 48, 8320), ("token64", "gemv", 5, 48, 8320), ("token128", "gemv", 1, 48, 8192),
     ("token128", "gemv", 2, 8192, 8320), ("token128", "gemv", 1, 8208, 8320),
-    ("w8", "gemm", 8, 117984, 4608), ("w8", "gemm", 9, 117984, 4608), ("w8", "gemv", 1, 131072, 4608)])
+    ("w8", "gemm", 8, 117984, 4608), ("w8", "gemm", 9, 117984, 4608), ("w8", "gemv", 1, 131072, 4608),
+    # one and two splits of one or two tokens, four splits, sixteen splits on
+    # either side of the K-parallel kernel's slices, K past its LDS, reference
+    # mode with many rows, and full rounds of W8 rows
+    ("token128", "gemm", 1, 32784, 2560), ("token128", "gemm", 2, 20496, 2432), ("token64", "gemm", 2, 8192, 4096),
+    ("token64", "gemm", 2, 8208, 4096), ("token64", "gemm", 8, 14336, 6144), ("token64", "gemm", 12, 6144, 4608),
+    ("token64", "gemm", 8, 592, 7936), ("token64", "gemm", 8, 640, 6144), ("token64", "gemm", 4, 3072, 17408),
+    ("token128", "gemm", 4, 1024, 1152), ("token128", "gemm", 5, 1024, 2176), ("token128", "gemv", 4, 4096, 4224),
+    ("token64", "gemm", 1, 48, 49280), ("token128", "gemm", 1, 48, 98432),
+    ("block64", "gemm", 4, 32784, 640), ("block64", "gemm", 2, 32784, 640), ("block32", "gemm", 8, 24576, 4096),
+    ("block64", "gemm", 8, 24592, 4096), ("block64", "gemv", 3, 65536, 384),
+    ("w8", "gemm", 9, 57344, 4608), ("w8", "gemm", 8, 57344, 4608), ("w8", "gemm", 2, 245760, 4608)])
 def test_strip_rowwave_line(mode, call, T, M, K):
     group, block, enc = MODES[mode]
     g = torch.Generator(device=DEV).manual_seed(T * M + K)
