@@ -27,6 +27,9 @@
 // that XCD's L2.
 #include "kxw4_device.hpp"
 #include "kxw4_internal.hpp"
+#include "kxw4_route.hpp"
+
+#include <algorithm>
 
 
 namespace kxw4 {
@@ -460,9 +463,80 @@ static long long strips_of(const StripArgs &s) {
     return n;
 }
 
+// Every split count runs on the strip kernel; what is planned with one split
+// goes to the large tiles where it fills them. Returns 1 (nothing launched)
+// where the general kernel is ahead.
+static int launch_planned(const GemmArgs &a, hipStream_t st) {
+    StripArgs split = strip_args(a, kVarGemm, 2, 16), one = strip_args(a, kVarGemm, 1, 1);
+    // runs of neighbouring segments whose one-split weights are the same, as
+    // projections of their own for the large tiles; the others (with too few
+    // strips for the tiles, or past their 32-bit offsets) share one launch
+    struct Run {
+        unsigned mask;
+        int s0, s1;
+    } runs[kMaxSegments];
+    int nruns = 0;
+    StripArgs rest = one;
+    if (strips_of(one) > strip_limit(a)) {
+        auto ones = [&](int s) {
+            unsigned m = 0;
+            for (int i = 0; i < a.count; ++i) m |= (unsigned)(a.w[i].seg_split[s] == 1) << i;
+            return m;
+        };
+        rest.entries = 0;
+        for (int s0 = 0, s1; s0 < a.seg_count; s0 = s1) {
+            const unsigned m = ones(s0);
+            for (s1 = s0 + 1; s1 < a.seg_count && ones(s1) == m; ++s1) {}
+            if (!m) continue;
+            const int t0 = s0 ? a.seg_end[s0 - 1] : 0, t1 = a.seg_end[s1 - 1];
+            StripArgs run = one;
+            run.entries = 0;
+            for (int i = 0; i < one.entries; ++i) {
+                StripEntry e = one.e[i];                     // (an entry may reach over several runs)
+                e.t0 = std::max(e.t0, t0);
+                e.t1 = std::min(e.t1, t1);
+                if (e.t0 < e.t1) run.e[run.entries++] = e;
+            }
+            if (strips_of(run) > strip_limit(a)) runs[nruns++] = Run{m, s0, s1};
+            else for (int i = 0; i < run.entries; ++i) rest.e[rest.entries++] = run.e[i];
+        }
+    }
+    if (a.block == 0 && split.entries && one.entries) {
+        PackedShape p{device_cus(), a.K, a.group, nruns + (rest.entries != 0), nruns, 0, 0, strips_of(rest), 0, 0};
+        for (int i = 0; i < split.entries; ++i) {
+            const int t = split.e[i].t1 - split.e[i].t0, rgs = split.w[split.e[i].w].M / 16;
+            (t <= 8 ? p.few : p.lots) += (long long)rgs * ((t + 15) / 16);
+        }
+        p.launches += (p.few != 0) + (p.lots != 0);
+        for (int i = 0; i < a.count; ++i) {
+            const int rgs = a.w[i].M / 16;
+            p.general += (long long)((rgs + 7) / 8) * ((a.T + 63) / 64);
+            for (int r = 0; r < nruns; ++r)
+                if (runs[r].mask >> i & 1)
+                    p.tile_work += (long long)rgs * (a.seg_end[runs[r].s1 - 1] - (runs[r].s0 ? a.seg_end[runs[r].s0 - 1] : 0));
+        }
+        if (packed_general(p)) return 1;
+    }
+    if (split.entries) {
+        const int r = launch_strip(split, st);
+        if (r) return r;
+    }
+    for (int i = 0; i < nruns; ++i) {
+        GemmArgs g = sub_gemm(a, runs[i].mask, runs[i].s0, runs[i].s1);
+        int r = launch_gemm3(g, st);
+        if (r == 1) r = launch_gemmr(g, st);
+        if (r == 1) {                                        // (past the tiles' offsets)
+            StripArgs s = strip_args(g, kVarGemm, 1, 1);
+            r = launch_strip(s, st);
+        }
+        if (r) return r;
+    }
+    return rest.entries ? launch_strip(rest, st) : 0;
+}
+
 int launch_gemm(GemmArgs &a, bool debug, hipStream_t st) {
-    // Every split count runs on the strip kernel; what is planned with one
-    // split goes to the large tiles where it fills them (per-token: gemm3;
+    // The modes of the strip kernel go through launch_planned, the others to
+    // the large tiles where they are planned with one split (per-token: gemm3;
     // K32 activation blocks: gemmr). The gemm_kernel option keeps everything
     // here (the tests cover both), a gemm3_tile / gemmr_tile option asks for
     // the large tiles.
@@ -474,35 +548,8 @@ int launch_gemm(GemmArgs &a, bool debug, hipStream_t st) {
             r = launch_gemmr(a, st);
             if (r != 1) return r;
         } else {
-            StripArgs split = strip_args(a, kVarGemm, 2, 16);
-            if (split.entries) {
-                const int r = launch_strip(split, st);
-                if (r) return r;
-            }
-            StripArgs one = strip_args(a, kVarGemm, 1, 1);
-            if (!one.entries) return 0;
-            if (strips_of(one) <= strip_limit(a)) return launch_strip(one, st);
-            // runs of neighbouring segments whose one-split weights are the same
-            auto ones = [&](int s) {
-                unsigned m = 0;
-                for (int i = 0; i < a.count; ++i) m |= (unsigned)(a.w[i].seg_split[s] == 1) << i;
-                return m;
-            };
-            for (int s0 = 0, s1; s0 < a.seg_count; s0 = s1) {
-                const unsigned m = ones(s0);
-                for (s1 = s0 + 1; s1 < a.seg_count && ones(s1) == m; ++s1) {}
-                if (!m) continue;
-                GemmArgs g = sub_gemm(a, m, s0, s1);
-                StripArgs s = strip_args(g, kVarGemm, 1, 1);
-                int r = 1;
-                if (strips_of(s) > strip_limit(g)) {
-                    r = launch_gemm3(g, st);
-                    if (r == 1) r = launch_gemmr(g, st);
-                }
-                if (r == 1) r = launch_strip(s, st);         // (few strips, or past the large tiles' 32-bit offsets)
-                if (r) return r;
-            }
-            return 0;
+            const int r = launch_planned(a, st);
+            if (r != 1) return r;
         }
     }
     bool splits = false;

@@ -1,7 +1,8 @@
 // kxw4_route.hpp — which kernel a decode launch (at most 16 tokens) runs on:
 // the strip kernel (kxw4_strip.hip), the row-wave kernel (kxw4_rowwave.hip)
-// or the K-parallel kernel (kxw4_decode.hip). Plain C++, so that the rule can
-// be checked without a GPU.
+// or the K-parallel kernel (kxw4_decode.hip); and, last, which packed prompts
+// run on the general GEMM kernel (kxw4_gemm.hip). Plain C++, so that the rules
+// can be checked without a GPU.
 //
 // Every kernel gives the same bits; the lines lie where the times cross. They
 // were measured over 256-73,728 rows (W8: 262,144) of 1,024-17,408 columns
@@ -121,6 +122,40 @@ inline DecodeRoute decode_route(const DecodeShape &s) {
     if (s.T > 16 || s.S == 0) return kRouteStrip;
     if (s.w8) return route_w8(s);
     return s.blocks ? route_blocks(s) : route_token(s);
+}
+
+// A packed prompt in per-token mode whose segments have one split and several:
+// strips and large tiles in a launch each, or the general GEMM kernel in one.
+struct PackedShape {
+    int cus, K, group;
+    int launches;                     // of the strip and large-tile kernels
+    int tile_runs;                    // of the large tiles
+    long long few, lots;              // split strips of at most 8 tokens, of 16
+    long long strips;                 // one-split strips of 32 tokens
+    long long tile_work;              // row-groups x tokens on the large tiles
+    long long general;                // work-groups (64 tokens x 128 rows) of the general kernel
+};
+
+// The general kernel's tiles reach over segments, so segments of a few tokens
+// cost it nothing, and it walks all of K in one pass whatever the split
+// counts: about 8 us per 1,000 columns while its work-groups are resident
+// (two per CU), more rows and tokens on top. The other launches cost their
+// strips and about 6 us each. Both sides fitted over 1,581 random packings of
+// 2-7 segments of 1-600 tokens, 512-17,408 rows, 1,024-17,408 columns (mean
+// error 9 %); us a projection, in thousands of columns. (123 + 48 + 119 + 33 +
+// 6 + 39 tokens of two weights of 5,344 rows, K = 1920, group 64: 54.8 against
+// 37.3 us on the general kernel; 16 + 32 + 64 + 128 + 256 tokens of two of
+// 5,120, K = 17408: 234 against 296.)
+inline bool packed_general(const PackedShape &s) {
+    const bool g64 = s.group == 64;
+    const double k = s.K / 1000.0, full = 2.0 * s.cus;
+    double general = 18 + k * (g64 ? 7.2 : 6.4);
+    if (s.general > s.cus) general += 2 * k;
+    if (s.general > full) general += k * (4.7 + (g64 ? 10.5 : 9.0) * (s.general / full - 1));
+    const double others = 5.6 * s.launches +
+                          k * ((1.0 * s.few + 1.5 * s.lots + 1.0 * s.strips) / 1000 + (s.strips ? 1.0 : 0.0) +
+                               2.5 * s.tile_runs + (g64 ? 3.0 : 2.0) * s.tile_work / 1e5);
+    return others > general;
 }
 
 }  // namespace kxw4

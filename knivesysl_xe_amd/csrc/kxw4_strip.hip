@@ -596,26 +596,73 @@ static int st_rw(StripArgs &a, int T, int smax, hipStream_t st) {
     }
 }
 
+// Whether the entries of split count SC fill 32-token tiles: these share a
+// row-group's unpack and scales between two blocks and
+// pay once the 16-token ones fill the SIMDs four times over (W8, with no
+// unpack but twice the weight bytes: twice) and their padding costs less than
+// that (a 32-token strip takes 1.6 times a 16-token one).
+static bool st_fills_32(const StripArgs &a, int SC, int per_simd) {
+    long long strips16 = 0, strips32 = 0;
+    for (int i = 0; i < a.entries; ++i) {
+        if (a.e[i].S != SC) continue;
+        const long long t = a.e[i].t1 - a.e[i].t0, rgs = a.w[a.e[i].w].M / 16;
+        strips16 += rgs * ((t + 15) / 16);
+        strips32 += rgs * ((t + 31) / 32);
+    }
+    return strips16 * SC > per_simd && 5 * strips16 > 8 * strips32;
+}
+
+// The entries of `a` that `pick` names, taken out of it.
+template <class F>
+static StripArgs st_take(StripArgs &a, F pick) {
+    StripArgs own = a;
+    int left = 0;
+    own.entries = 0;
+    for (int i = 0; i < a.entries; ++i) {
+        if (pick(a.e[i])) own.e[own.entries++] = a.e[i];
+        else a.e[left++] = a.e[i];
+    }
+    a.entries = left;
+    return own;
+}
+
 template <int UNIT, bool BLK, int VAR, int WF>
 static int st_shape(StripArgs &a, hipStream_t st) {
+    constexpr int kFill = WF == kStW8 ? 2000 : 4400;
     int T = 0, smax = 1;
-    long long strips16 = 0, strips32 = 0;
     a.same_s = 1;
     for (int i = 0; i < a.entries; ++i) {
-        const int t = a.e[i].t1 - a.e[i].t0, rgs = a.w[a.e[i].w].M / 16;
-        T = std::max(T, t);
+        T = std::max(T, a.e[i].t1 - a.e[i].t0);
         smax = std::max(smax, a.e[i].S);
         a.same_s &= a.e[i].S == a.e[0].S;
-        strips16 += (long long)rgs * ((t + 15) / 16);
-        strips32 += (long long)rgs * ((t + 31) / 32);
     }
-    // 32-token tiles share a row-group's unpack and scales between two
-    // blocks; they pay once the 16-token ones fill the SIMDs four times over
-    // (W8, with no unpack but twice the weight bytes: twice) and their
-    // padding costs less than that (a 32-token strip takes 1.6 times a
-    // 16-token one)
-    if (smax <= 4 && a.same_s && strips16 * smax > (WF == kStW8 ? 2000 : 4400) && 5 * strips16 > 8 * strips32)
-        return st_rw<32, UNIT, BLK, VAR, WF>(a, T, smax, st);
+    if (a.same_s) {
+        if (smax <= 4 && st_fills_32(a, smax, kFill)) return st_rw<32, UNIT, BLK, VAR, WF>(a, T, smax, st);
+    } else {
+        // entries of one split count that fill the 32-token tiles by
+        // themselves: a launch of their own
+        for (int SC = 1; SC <= 4; SC *= 2) {
+            if (!st_fills_32(a, SC, kFill)) continue;
+            StripArgs rest = a;
+            StripArgs own = st_take(rest, [&](const StripEntry &e) { return e.S == SC; });
+            const int r = st_shape<UNIT, BLK, VAR, WF>(own, st);
+            return r ? r : st_shape<UNIT, BLK, VAR, WF>(rest, st);
+        }
+        // few-token entries apart from the others, once the grid is several
+        // rounds deep: a 16-token tile of theirs costs as much as a full one
+        // (1 + 1 + 14 + 19 + 34 tokens of two weights of 3,568 rows, K = 3712,
+        // beside 371 tokens in one split: 103 -> 80 us; a shallower grid only
+        // pays the second launch)
+        StripArgs rest = a;
+        StripArgs few = st_take(rest, [](const StripEntry &e) { return e.t1 - e.t0 <= 8; });
+        long long strips16 = 0;
+        for (int i = 0; i < a.entries; ++i)
+            strips16 += (long long)(a.w[a.e[i].w].M / 16) * ((a.e[i].t1 - a.e[i].t0 + 15) / 16);
+        if (few.entries && rest.entries && strips16 > 6ll * device_cus()) {
+            const int r = st_shape<UNIT, BLK, VAR, WF>(few, st);
+            return r ? r : st_shape<UNIT, BLK, VAR, WF>(rest, st);
+        }
+    }
     if (T == 1) return st_rw<1, UNIT, BLK, VAR, WF>(a, T, smax, st);
     if (T == 2) return st_rw<2, UNIT, BLK, VAR, WF>(a, T, smax, st);
     if (T <= 8) return st_rw<8, UNIT, BLK, VAR, WF>(a, T, smax, st);

@@ -54,6 +54,18 @@ def check(y, ref, what):
     assert np.array_equal(got, ref.view(bits)), f"{what}: {np.count_nonzero(got != ref.view(bits))} of {got.size} differ"
 
 
+def launches(call):
+    """Kernel launches of `call`, counted as the nodes of its captured graph."""
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        call()
+    n = C.c_size_t()
+    assert C.CDLL(path).hipGraphGetNodes(C.c_void_p(g.raw_cuda_graph()), None, C.byref(n)) == 0
+    return n.value
+
+
 # tokens around the tile sizes (1, 2, 8, 16, 32); one K tile, an odd number of
 # tiles (a half-empty last stage) and enough for whole stages; row-groups that
 # do not divide the row waves; splits that end inside a tile (K = 640: 20 K32
@@ -98,8 +110,8 @@ def test_strip_gemv(mode, T, M, K, splits):
 
 
 # packed prompts whose segments have different split counts, and weights of a
-# fan-out that are planned apart: strips of several split counts beside the
-# large tiles, over token ranges that start and end anywhere
+# fan-out that are planned apart: strips of several split counts, over token
+# ranges that start and end anywhere
 @pytest.mark.parametrize("mode", ["token128", "token64", "block32", "w8"])
 @pytest.mark.parametrize("rows,segs", [([4096], [9, 61, 300, 5]), ([8192, 48], [70, 3, 129]), ([1024, 2048], [250, 17, 40])])
 def test_strip_packed_segments(mode, rows, segs):
@@ -155,18 +167,6 @@ def test_strip_rowwave_line(mode, call, T, M, K):
         check(y[:, lo:lo + 48].contiguous(), oracle(mode, c, s, act, var, sp), f"{mode} {call} T={T} M={M} K={K} row {lo}")
 
 
-def launches(call):
-    """Kernel launches of `call`, counted as the nodes of its captured graph."""
-    with open("/proc/self/maps") as f:
-        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
-    g = torch.cuda.CUDAGraph(keep_graph=True)
-    with torch.cuda.graph(g):
-        call()
-    n = C.c_size_t()
-    assert C.CDLL(path).hipGraphGetNodes(C.c_void_p(g.raw_cuda_graph()), None, C.byref(n)) == 0
-    return n.value
-
-
 # long K at 8 and 16 tokens: the row-wave kernel's LDS does not hold the
 # activations, and one launch that reads the weight once takes all of them
 @pytest.mark.parametrize("mode,T", [("w8", 8), ("w8", 16), ("k16", 8), ("k16", 16)])
@@ -182,3 +182,72 @@ def test_long_k_reads_the_weight_once(mode, T):
             y = ops.gemv(w, a)
             check(y, want, f"{mode} T={T}")
             assert launches(lambda: ops.gemv(w, a, out=y)) == 1
+
+
+# Packed prompts past the strip kernel's limit: split segments on the strips,
+# each run of one-split segments on the large tiles as a projection of its own
+# (t0 > 0, weights left out, residual and BF16 rows shifted with it), what is
+# too small for the tiles in one strip launch, few-token entries apart from the
+# others in a deep grid, split counts that fill 32-token tiles apart, and plans
+# that the general kernel takes in one launch. `n` is the launches that shows
+# which way a plan went; the first and last rows go against the oracle.
+@pytest.mark.parametrize("mode,rows,K,segs,n", [
+    ("token64", [8192], 384, [3, 700, 5, 600], 3), ("token128", [8192], 384, [3, 700, 5, 600], 3),
+    ("block32", [8192], 384, [3, 700, 5, 600], 3), ("block64", [8192], 384, [9, 700, 5, 600], 3),
+    ("token64", [1024, 32768], 1024, [200, 400, 230], 4), ("block32", [1024, 32768], 384, [200, 400, 230], 4),
+    ("token128", [1024, 32768], 1024, [200, 400, 230], 4),
+    ("block32", [3568, 3568], 384, [34, 1, 121, 250, 19, 14, 1], 3),
+    ("token64", [5344, 5344], 1920, [123, 48, 119, 33, 6, 39], 1),
+    ("token128", [9008, 9008], 4096, [100, 1, 100, 1, 100], 1),
+    ("token128", [8192], 384, [20, 20, 20, 20, 3], 2), ("block32", [8192], 384, [20, 20, 20, 20, 3], 2),
+    ("w8", [8192], 384, [20, 20, 20, 20, 3], 2)])
+def test_packed_beside_the_large_tiles(mode, rows, K, segs, n):
+    group, block, enc = MODES[mode]
+    g = torch.Generator(device=DEV).manual_seed(sum(rows) + sum(segs))
+    lim = (-128, 128) if mode == "w8" else (-8, 8)
+    T, off = sum(segs), [0] + [int(o) for o in np.cumsum(segs)]
+    ws = []
+    for M in rows:
+        codes = torch.randint(*lim, (M, K), generator=g, device=DEV, dtype=torch.int8)
+        bits = (0.02 * torch.rand(M, K // group, generator=g, device=DEV)).to(torch.float16).view(torch.int16)
+        w = ops.W4Weight.from_codes_s8(codes, bits) if mode == "w8" else ops.W4Weight.from_codes(codes, bits, group, enc)
+        ws.append((codes, bits, w))
+    x = torch.randn(T, K, generator=g, device=DEV).cpu().numpy()
+    a, act = ops.quantize_act(dev(x), block), O.quantize_act(x, block)
+    res = torch.randn(T, rows[0], generator=g, device=DEV)
+    for out in (torch.float32, torch.bfloat16):
+        if len(rows) == 1:
+            y = ops.gemm(ws[0][2], a, out, residual=res, offsets=off)
+            assert launches(lambda: ops.gemm(ws[0][2], a, out, residual=res, offsets=off, out=y)) == n
+            ys = [y]
+        else:
+            ys = ops.gemm_fanout([w for _, _, w in ws], a, out, offsets=off)
+            assert launches(lambda: ops.gemm_fanout([w for _, _, w in ws], a, out, offsets=off, outs=ys)) == n
+        for (codes, bits, _), y in zip(ws, ys):
+            M = codes.shape[0]
+            sp = O.segment_splits(T, M, K, off)
+            for lo in (0, M - 48):
+                c, s = codes[lo:lo + 48].cpu().numpy(), bits[lo:lo + 48].cpu().numpy().view(np.uint16)
+                kw = {"residual": res[:, lo:lo + 48].contiguous().cpu().numpy()} if len(rows) == 1 else {}
+                check(y[:, lo:lo + 48].contiguous(),
+                      oracle(mode, c, s, act, O.VAR_GEMM, sp, out_bf16=out == torch.bfloat16, **kw),
+                      f"{mode} rows={M} from {lo} {out}")
+
+
+# 32-token tiles of two and four splits, a partial last tile, with residual
+@pytest.mark.parametrize("mode", ["token128", "token64", "block32", "block64", "w8"])
+@pytest.mark.parametrize("forced", [2, 4])
+def test_strip_split_32_token_tiles(mode, forced):
+    M, K, T = 8192, 640, 70
+    rng = np.random.default_rng(forced)
+    codes, scales, w = weight(rng, mode, M, K)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    res = rng.standard_normal((T, M)).astype(np.float32)
+    block = MODES[mode][1]
+    a, act = ops.quantize_act(dev(x), block), O.quantize_act(x, block)
+    sp = O.segment_splits(T, M, K, None, forced)
+    y = ops.gemm(w, a, residual=dev(res), forced_splits=forced)
+    for lo in (0, M - 48):
+        check(y[:, lo:lo + 48].contiguous(),
+              oracle(mode, codes[lo:lo + 48], scales[lo:lo + 48], act, O.VAR_GEMM, sp,
+                     residual=np.ascontiguousarray(res[:, lo:lo + 48])), f"{mode} forced {forced} rows from {lo}")

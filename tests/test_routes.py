@@ -16,16 +16,28 @@ CUS = 256
 
 
 @pytest.fixture(scope="module")
-def route(tmp_path_factory):
+def rules(tmp_path_factory):
     d = tmp_path_factory.mktemp("route")
     src, out = d / "route.cpp", d / "route.so"
     src.write_text('#include "kxw4_route.hpp"\n'
                    'extern "C" int route(int rgs, int T, int K, int group, int S, int blocks, int w8) {\n'
                    f'    return kxw4::decode_route({{{CUS}, rgs, T, K, group, S, blocks != 0, w8 != 0}});\n'
+                   '}\n'
+                   'extern "C" int packed(int K, int group, int launches, int tile_runs, long long few, long long lots,\n'
+                   '                      long long strips, long long tile_work, long long general) {\n'
+                   f'    return kxw4::packed_general({{{CUS}, K, group, launches, tile_runs, few, lots, strips, tile_work,'
+                   ' general});\n'
                    '}\n')
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I", CSRC, str(src), "-o", str(out)],
                    check=True)
-    return C.CDLL(str(out)).route
+    lib = C.CDLL(str(out))
+    lib.packed.argtypes = [C.c_int] * 4 + [C.c_longlong] * 5
+    return lib.route, lib.packed
+
+
+@pytest.fixture(scope="module")
+def route(rules):
+    return rules[0]
 
 
 def splits(call, M, K, T):
@@ -103,3 +115,33 @@ def test_other_plans_stay_on_the_strips(route):
     assert route(2176, 17, 5120, 128, 1, 0, 0) == STRIP      # more than 16 tokens
     assert route(2176, 8, 5120, 128, 0, 0, 0) == STRIP       # split counts that differ
     assert route(320, 1, 17408, 16, 8, 1, 0) == STRIP        # K16
+
+
+# (rows of each weight, K, segments; us on the strips and tiles / on the general kernel)
+@pytest.mark.parametrize("group,rows,K,segs,want", [
+    (64, [5344, 5344], 1920, [123, 48, 119, 33, 6, 39], True),           # 54.8 / 37.3
+    (128, [9008, 9008], 4096, [100, 1, 100, 1, 100], True),              # 100 / 75
+    (128, [17408], 5120, [100, 1, 100, 1, 100], True),                   # 120 / 95
+    (64, [7952, 7952], 12160, [132, 7, 6, 34], True),                    # 189 / 136
+    (128, [1968], 8192, [154, 5], False),                                # 25 / 64
+    (64, [5120], 5120, [16, 32, 64, 128, 256], False),                   # 45 / 64
+    (64, [5120, 5120], 17408, [16, 32, 64, 128, 256], False),            # 234 / 296
+    (128, [9008, 9008], 4096, [16, 32, 64, 128, 256], False),            # 64 / 113
+    (64, [9968], 4352, [14, 239, 239], False),                           # 62 / 88
+])
+def test_packed_prompts(rules, group, rows, K, segs, want):
+    rgs, limit = [M // 16 for M in rows], 4000
+    S = [int(O.gemm_splits(rgs[0], (t + 7) // 8, K // 32, 0)) for t in segs]
+    runs, open_ = [], False
+    for t, s in zip(segs, S):
+        if s == 1:
+            runs = runs[:-1] + [runs[-1] + t] if open_ else runs + [t]
+        open_ = s == 1
+    strips = lambda t: sum(rgs) * -(-t // 32)
+    tiles = [t for t in runs if strips(t) > limit] if sum(map(strips, runs)) > limit else []
+    rest = sum(strips(t) for t in runs if t not in tiles)
+    few = sum(sum(rgs) for t, s in zip(segs, S) if s > 1 and t <= 8)
+    lots = sum(sum(rgs) * -(-t // 16) for t, s in zip(segs, S) if s > 1 and t > 8)
+    launches = len(tiles) + (rest > 0) + (few > 0) + (lots > 0)
+    general = sum(-(-r // 8) for r in rgs) * -(-sum(segs) // 64)
+    assert bool(rules[1](K, group, launches, len(tiles), few, lots, rest, sum(rgs) * sum(tiles), general)) == want
