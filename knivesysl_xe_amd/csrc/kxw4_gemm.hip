@@ -445,17 +445,8 @@ static GemmArgs sub_gemm(const GemmArgs &a, unsigned mask, int s0, int s1) {
     return g;
 }
 
-// One-split projections of up to this many 16-row x 32-token strips run on
-// the strip kernel, whose grid still fills the chip where the large tiles
-// leave CUs idle (per-token N = 5120, K = 17408, T = 256, 2,560 strips: 58
-// against 81 us; N = 17408, K = 5120, T = 128, 4,352 strips: 35 against 35
-// us, T = 256: 53 against 46; block mode N = 5120, K = 17408, T = 512, 5,120
-// strips: 227 against 234 us, N = 17408, K = 5120, T = 256, 8,704 strips: 113
-// against 109 us). W8 has no large-tile kernel, so all of it goes there.
-static long long strip_limit(const GemmArgs &a) {
-    if (a.w8) return 1ll << 62;
-    return a.block == 32 ? 5500 : 4000;
-}
+// W8 has no large-tile kernel, so all of it runs on strips.
+static long long strip_limit(const GemmArgs &a) { return a.w8 ? 1ll << 62 : one_split_strips(a.block, a.group); }
 
 static long long strips_of(const StripArgs &s) {
     long long n = 0;

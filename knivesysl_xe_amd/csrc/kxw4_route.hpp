@@ -124,6 +124,20 @@ inline DecodeRoute decode_route(const DecodeShape &s) {
     return s.blocks ? route_blocks(s) : route_token(s);
 }
 
+// One-split projections of up to this many 16-row x 32-token strips run on
+// the strip kernel, whose grid still fills the chip where the large tiles
+// leave CUs idle (us on strips / on tiles). Per token, group 128: N = 5120, K =
+// 17408, T = 256, 2,560 strips: 58 / 81; up to 4,000 strips 10-30 % ahead. Group
+// 64, whose tiles share more of the unpack: up to 3,100 strips 9 % ahead, from
+// there to 4,000 2 % behind (17,408 rows, K = 5120, T = 96, 3,264 strips: 33.1 /
+// 29.8; 14,336 rows, K = 4096, T = 128: 27.0 / 24.9). Reference mode: N = 5120,
+// K = 17408, T = 512, 5,120 strips: 227 / 234; 17,408 rows, K = 5120, T = 256,
+// 8,704 strips: 113 / 109.
+inline long long one_split_strips(int block, int group) {
+    if (block == 32) return 5500;
+    return group == 64 ? 3100 : 4000;
+}
+
 // A packed prompt in per-token mode whose segments have one split and several:
 // strips and large tiles in a launch each, or the general GEMM kernel in one.
 struct PackedShape {

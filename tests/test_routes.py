@@ -27,17 +27,19 @@ def rules(tmp_path_factory):
                    '                      long long strips, long long tile_work, long long general) {\n'
                    f'    return kxw4::packed_general({{{CUS}, K, group, launches, tile_runs, few, lots, strips, tile_work,'
                    ' general});\n'
-                   '}\n')
+                   '}\n'
+                   'extern "C" long long limit(int block, int group) { return kxw4::one_split_strips(block, group); }\n')
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I", CSRC, str(src), "-o", str(out)],
                    check=True)
     lib = C.CDLL(str(out))
     lib.packed.argtypes = [C.c_int] * 4 + [C.c_longlong] * 5
-    return lib.route, lib.packed
+    lib.limit.restype = C.c_longlong
+    return lib
 
 
 @pytest.fixture(scope="module")
 def route(rules):
-    return rules[0]
+    return rules.route
 
 
 def splits(call, M, K, T):
@@ -130,7 +132,7 @@ def test_other_plans_stay_on_the_strips(route):
     (64, [9968], 4352, [14, 239, 239], False),                           # 62 / 88
 ])
 def test_packed_prompts(rules, group, rows, K, segs, want):
-    rgs, limit = [M // 16 for M in rows], 4000
+    rgs, limit = [M // 16 for M in rows], rules.limit(0, group)
     S = [int(O.gemm_splits(rgs[0], (t + 7) // 8, K // 32, 0)) for t in segs]
     runs, open_ = [], False
     for t, s in zip(segs, S):
@@ -144,4 +146,19 @@ def test_packed_prompts(rules, group, rows, K, segs, want):
     lots = sum(sum(rgs) * -(-t // 16) for t, s in zip(segs, S) if s > 1 and t > 8)
     launches = len(tiles) + (rest > 0) + (few > 0) + (lots > 0)
     general = sum(-(-r // 8) for r in rgs) * -(-sum(segs) // 64)
-    assert bool(rules[1](K, group, launches, len(tiles), few, lots, rest, sum(rgs) * sum(tiles), general)) == want
+    assert bool(rules.packed(K, group, launches, len(tiles), few, lots, rest, sum(rgs) * sum(tiles), general)) == want
+
+
+# one split: strips or large tiles (us on strips / on tiles)
+@pytest.mark.parametrize("block,group,M,T,strips", [
+    (0, 64, 17408, 96, False),                           # K = 5120: 33.1 / 29.8
+    (0, 64, 14336, 128, False),                          # K = 4096: 27.0 / 24.9
+    (0, 64, 10000, 192, False),                          # K = 1152: 13.2 / 11.4
+    (0, 64, 5120, 256, True),                            # K = 17408
+    (0, 128, 5120, 384, True),
+    (0, 128, 17408, 128, False),                         # K = 5120: 35 / 35
+    (32, 32, 5120, 512, True),                           # K = 17408: 227 / 234
+    (32, 64, 17408, 256, False),                         # K = 5120: 113 / 109
+])
+def test_one_split_strips(rules, block, group, M, T, strips):
+    assert (M // 16 * -(-T // 32) <= rules.limit(block, group)) == strips
