@@ -31,6 +31,7 @@
 //     ring of NST stages, one barrier per step.
 #include "kxw4_device.hpp"
 #include "kxw4_internal.hpp"
+#include "kxw4_route.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -489,11 +490,9 @@ static int launch_gr(GemmArgs &a, hipStream_t st) {
 // scales (graph replay, bit-exact, T=2048 K=N=5120 group 32 / T=512 K=17408
 // N=5120 group 64):
 //   4: 128 x 64, 4 waves of 2 token blocks, four work-groups per CU:
-//     191 / 264 us (the default while its grid gives every CU at least two
-//     work-groups: N=17408 K=5120 T=300 109 against 129 us for tile 9, N=5120
-//     T=384 with less than one 67 against 59);
-//   9: 128 x 32, 4 waves of one token block: 217 / 234 us (the default for
-//     smaller grids);
+//     191 / 264 us;
+//   9: 128 x 32, 4 waves of one token block: 217 / 234 us (4 or 9, whichever
+//     loads the busiest CU less: gemmr_wide in kxw4_route.hpp);
 //   0: 160 x 256, 10 waves of 4 token blocks (3, 3, 2, 2 per SIMD), one
 //     work-group per CU: 187 / 586 us;
 //   5: 160 x 64, 10 waves of one token block: 281 / 221 us;
@@ -531,10 +530,9 @@ int launch_gemmr(GemmArgs &a, hipStream_t st) {
     }
     int sel = options().gemmr_tile;
     if (sel < 0) {
-        long long tiles = 0;
-        for (int i = 0; i < a.count; ++i) tiles += (a.w[i].M / 16 + 7) / 8;
-        tiles *= (a.T + 63) / 64;
-        sel = tiles >= 2LL * device_cus() ? 4 : 9;
+        long long rows = 0;                                          // 128-row tiles
+        for (int i = 0; i < a.count; ++i) rows += (a.w[i].M / 16 + 7) / 8;
+        sel = gemmr_wide(device_cus(), rows, a.T) ? 4 : 9;
     }
     const bool zp = a.scale_enc == 1;
     switch (a.group) {

@@ -138,6 +138,18 @@ inline long long one_split_strips(int block, int group) {
     return group == 64 ? 3100 : 4000;
 }
 
+// Reference-mode GEMM tiles of 128 rows: 64 tokens wide, or 32. The wider one
+// takes a CU 1.65 times as long for twice the work (swept at 484 points: 1.56
+// to 1.84), so what counts is how many of each the busiest CU gets. 34,816
+// rows, K = 5120, T = 90: 3 wide against 4 narrow per CU, 111 against 92 us; T =
+// 128: 3 against 5, 112 / 116; 17,408 rows, T = 300: 3 against 6, 111 / 131;
+// 10,240 rows, T = 300: 2 against 4, 83 / 90. `rows`: 128-row tiles over all
+// weights.
+inline bool gemmr_wide(int cus, long long rows, int T) {
+    const long long wide = (rows * ((T + 63) / 64) + cus - 1) / cus, narrow = (rows * ((T + 31) / 32) + cus - 1) / cus;
+    return 165 * wide < 100 * narrow;
+}
+
 // A packed prompt in per-token mode whose segments have one split and several:
 // strips and large tiles in a launch each, or the general GEMM kernel in one.
 struct PackedShape {

@@ -28,12 +28,16 @@ def rules(tmp_path_factory):
                    f'    return kxw4::packed_general({{{CUS}, K, group, launches, tile_runs, few, lots, strips, tile_work,'
                    ' general});\n'
                    '}\n'
+                   'extern "C" int wide(long long rows, int T) {\n'
+                   f'    return kxw4::gemmr_wide({CUS}, rows, T);\n'
+                   '}\n'
                    'extern "C" long long limit(int block, int group) { return kxw4::one_split_strips(block, group); }\n')
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I", CSRC, str(src), "-o", str(out)],
                    check=True)
     lib = C.CDLL(str(out))
     lib.packed.argtypes = [C.c_int] * 4 + [C.c_longlong] * 5
     lib.limit.restype = C.c_longlong
+    lib.wide.argtypes = [C.c_longlong, C.c_int]
     return lib
 
 
@@ -162,3 +166,19 @@ def test_packed_prompts(rules, group, rows, K, segs, want):
 ])
 def test_one_split_strips(rules, block, group, M, T, strips):
     assert (M // 16 * -(-T // 32) <= rules.limit(block, group)) == strips
+
+
+# 64-token tiles or 32-token ones of the reference-mode GEMM, by the ratio of
+# their times (64 / 32) measured at K = 5120
+@pytest.mark.parametrize("M,T,wide", [
+    (34816, 90, False),                                  # 1.20
+    (17408, 210, False),                                 # 1.21
+    (6544, 600, False),                                  # 1.17
+    (8192, 384, False),                                  # 1.09
+    (10240, 300, True),                                  # 0.92
+    (17408, 300, True),                                  # 0.85
+    (17408, 512, True),                                  # 0.92-0.96
+    (12288, 700, True),                                  # 0.93
+])
+def test_reference_mode_tiles(rules, M, T, wide):
+    assert bool(rules.wide((M // 16 + 7) // 8, T)) == wide
