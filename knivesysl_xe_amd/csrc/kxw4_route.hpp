@@ -150,6 +150,20 @@ inline bool gemmr_wide(int cus, long long rows, int T) {
     return 165 * wide < 100 * narrow;
 }
 
+// W4A4 GEMM tiles of 64 rows: 64 tokens, or 128. At K = 17408 a 64 x 64 tile
+// takes a CU 46-51 us and a 128 x 64 tile, whose two token blocks share the
+// weight unpack, 88-95 us: 1.87 times as long for twice the work, so the
+// smaller one wins where its finer grid saves more than that, and where two of
+// them run side by side in place of a single large one (swept at 284 points;
+// 64 x 64 against 128 x 64, N = 5120, K = 17408: T = 64 98 against 134 us, T = 512
+// 154.7 / 179.8, T = 1024 252 / 284, T = 2048 463 / 441; N = 17408, K = 5120, T =
+// 512 128.5 / 134.2; N = 2048, K = 5120, T = 1024, two for one: 40.2 / 42.7).
+// `rows`: 64-row tiles.
+inline bool w4a4_small(int cus, long long rows, int T) {
+    const long long large = (rows * ((T + 127) / 128) + cus - 1) / cus, small = (rows * ((T + 63) / 64) + cus - 1) / cus;
+    return large == 1 || 100 * small < 187 * large;
+}
+
 // A packed prompt in per-token mode whose segments have one split and several:
 // strips and large tiles in a launch each, or the general GEMM kernel in one.
 struct PackedShape {

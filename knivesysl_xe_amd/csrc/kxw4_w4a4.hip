@@ -26,6 +26,7 @@
 // NST stages.
 #include "kxw4_device.hpp"
 #include "kxw4_internal.hpp"
+#include "kxw4_route.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -410,24 +411,14 @@ static int launch_w4(W4a4Args &a, hipStream_t st) {
 }
 
 int launch_w4a4(W4a4Args &a, hipStream_t st) {
-    // 64 x 64 or 128 x 64, whichever loads the busiest CU less. At
-    // K = 17408 a 64 x 64 tile takes a CU 46-51 us and a 128 x 64 tile, whose
-    // two token blocks share the weight unpack, 88-95 us: 1.87 times as long
-    // for twice the work, so the smaller tile wins where its finer grid
-    // saves more than that. N = 5120, K = 17408, 64 x 64 against 128 x 64: T = 64
-    // 98 against 134 us, T = 512 154.7 / 179.8, T = 1024 252 / 284, T = 2048
-    // 463 / 441; N = 17408, K = 5120, T = 512 128.5 / 134.2. (128 x 64 at two
-    // or more work-groups per CU, as before, gave 171 us at T = 512 cold and
-    // 302 at T = 1024; 64 x 160 with 10 waves 197 at T = 512, since with one
-    // token block per wave the zero-point weight unpack is not shared.)
+    // 64 x 64 or 128 x 64, whichever loads the busiest CU less (w4a4_small in
+    // kxw4_route.hpp). (128 x 64 at two or more work-groups per CU, as before,
+    // gave 171 us at N = 5120, K = 17408, T = 512 cold and 302 at T = 1024; 64 x
+    // 160 with 10 waves 197 at T = 512, since with one token block per wave
+    // the zero-point weight unpack is not shared.)
     // the w4a4_tile option (0..4) picks one configuration (tests, tuning)
     int sel = options().w4a4_tile;
-    if (sel < 0) {
-        const long long cus = device_cus(), nt = (a.M / 16 + 3) / 4;
-        const long long big = (((a.T + 127) / 128) * nt + cus - 1) / cus;
-        const long long small = (((a.T + 63) / 64) * nt + cus - 1) / cus;
-        sel = 100 * small < 187 * big ? 4 : 0;
-    }
+    if (sel < 0) sel = w4a4_small(device_cus(), (a.M / 16 + 3) / 4, a.T) ? 4 : 0;
     switch (sel) {
     case 3: return launch_w4<1, 1, 2, 5, 3, 3>(a, st);      // 64 tokens x 160 rows, 10 waves
     case 1: return launch_w4<2, 1, 2, 4, 3, 2>(a, st);      // 128 tokens x 128 rows, 8 waves

@@ -31,13 +31,16 @@ def rules(tmp_path_factory):
                    'extern "C" int wide(long long rows, int T) {\n'
                    f'    return kxw4::gemmr_wide({CUS}, rows, T);\n'
                    '}\n'
+                   'extern "C" int small_tile(long long rows, int T) {\n'
+                   f'    return kxw4::w4a4_small({CUS}, rows, T);\n'
+                   '}\n'
                    'extern "C" long long limit(int block, int group) { return kxw4::one_split_strips(block, group); }\n')
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I", CSRC, str(src), "-o", str(out)],
                    check=True)
     lib = C.CDLL(str(out))
     lib.packed.argtypes = [C.c_int] * 4 + [C.c_longlong] * 5
     lib.limit.restype = C.c_longlong
-    lib.wide.argtypes = [C.c_longlong, C.c_int]
+    lib.wide.argtypes = lib.small_tile.argtypes = [C.c_longlong, C.c_int]
     return lib
 
 
@@ -182,3 +185,16 @@ def test_one_split_strips(rules, block, group, M, T, strips):
 ])
 def test_reference_mode_tiles(rules, M, T, wide):
     assert bool(rules.wide((M // 16 + 7) // 8, T)) == wide
+
+
+# 64 x 64 or 128 x 64 tiles of the W4A4 GEMM (us 64 x 64 / 128 x 64)
+@pytest.mark.parametrize("M,T,small", [
+    (5120, 64, True),                                    # K = 17408: 98 / 134
+    (5120, 512, True),                                   # 154.7 / 179.8
+    (5120, 2048, False),                                 # 463 / 441
+    (2048, 1024, True),                                  # K = 5120: 40.2 / 42.7
+    (8320, 84, True),                                    # K = 1408: 13.0 / 14.3
+    (4096, 1024, False),                                 # two large for four small: 1.07
+])
+def test_w4a4_tiles(rules, M, T, small):
+    assert bool(rules.small_tile((M // 16 + 3) // 4, T)) == small
