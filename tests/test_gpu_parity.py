@@ -421,17 +421,16 @@ def test_baseline_cfg4_row_subset():
 
 @pytest.fixture
 def kparallel():
-    # up to 16 tokens normally run on the row-wave kernel; this keeps the
-    # K-parallel decode kernel covered at the decode configurations
+    # few of these run on the K-parallel decode kernel by default; this keeps
+    # it covered at the decode configurations
     with ops.option("decode_kernel", 1):
         yield
 
 
 @pytest.fixture
 def rowwave():
-    # per-token shapes with at most 8 tokens and no more row-groups than CUs
-    # (cfg0, the small golden cases) normally run on the K-parallel kernel;
-    # this keeps the row-wave kernel covered there
+    # cfg0 and the small golden cases normally run on the strip or the
+    # K-parallel kernel; this keeps the row-wave kernel covered there
     with ops.option("decode_kernel", 2):
         yield
 
@@ -522,7 +521,7 @@ def test_decode_shapes(rows, K, T, group, block, enc, variant, forced):
 
 @pytest.fixture
 def gemm_general():
-    # the per-token prefill shapes normally run on the large-tile GEMM
+    # the per-token prefill shapes normally run on the strip or the large-tile
     # kernel; this keeps the general GEMM kernel covered on them
     with ops.option("gemm_kernel", 1):
         yield
@@ -578,6 +577,19 @@ def test_gemm3_auto_tile(rows, K, T, group):
     test_gemm3_shapes(rows, K, T, group, None)
 
 
+def strips(rows, T):
+    return sum(M // 16 for M in rows) * -(-T // 32)
+
+
+@pytest.mark.parametrize("rows,K,T,group", [
+    # the same past the strip kernel's limit (csrc/kxw4_route.hpp: at most
+    # 4,000 strips per token), where the default dispatch runs the chooser's pick
+    ([8192], 256, 300, 128), ([8208], 384, 280, 64), ([5120, 4112], 640, 250, 64), ([16400], 256, 97, 64)])
+def test_gemm3_auto_tile_past_the_strips(rows, K, T, group):
+    assert strips(rows, T) > 4000
+    test_gemm3_shapes(rows, K, T, group, None)
+
+
 @pytest.fixture(params=list(range(10)))
 def gemmr_tile(request):
     # every tile configuration of the reference-mode large-tile kernel
@@ -612,6 +624,16 @@ def test_gemmr_shapes(rows, K, T, group, enc, gemmr_tile):
     got = to_np(ops.gemm(ws[0], a, torch.bfloat16, residual=dev(res)))
     ref = O.project(*wts[0], group, enc, q, s, sm, 32, O.VAR_GEMM, sps[0], residual=res, out_bf16=True)
     assert_parity(got, ref, "bf16 + residual", bf16=True)
+
+
+@pytest.mark.parametrize("rows,K,T,group", [
+    # the default dispatch past the strip kernel's 5,500 strips, with the wide
+    # and the narrow tile the rule picks, ragged tokens and a fan-out
+    ([17408], 256, 180, 32), ([34816], 128, 90, 64), ([8208, 8192], 384, 200, 64), ([17424], 256, 210, 32)])
+def test_gemmr_auto_tile(rows, K, T, group):
+    assert strips(rows, T) > 5500
+    test_gemmr_shapes(rows, K, T, group, 1, None)
+
 
 
 def test_gemmr_packed_segments(gemmr_tile):

@@ -251,3 +251,43 @@ def test_strip_split_32_token_tiles(mode, forced):
         check(y[:, lo:lo + 48].contiguous(),
               oracle(mode, codes[lo:lo + 48], scales[lo:lo + 48], act, O.VAR_GEMM, sp,
                      residual=np.ascontiguousarray(res[:, lo:lo + 48])), f"{mode} forced {forced} rows from {lo}")
+
+
+# the modes that reach the other decode kernels by option only (decode_kernel:
+# 1 K-parallel, 2 row-wave), and the general GEMM's W8 path
+@pytest.mark.parametrize("kernel", [1, 2])
+@pytest.mark.parametrize("mode", ["block32", "block64", "w8", "k16"])
+@pytest.mark.parametrize("T,M,K,S", [(1, 80, 640, 16), (2, 48, 384, 1), (3, 144, 1152, 8), (8, 80, 640, 2), (9, 48, 384, 4),
+                                     (16, 144, 640, 8)])
+def test_other_decode_kernels(mode, kernel, T, M, K, S):
+    rng = np.random.default_rng(T * M + K + S)
+    codes, scales, w = weight(rng, mode, M, K)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    res = rng.standard_normal((T, M)).astype(np.float32)
+    a, act = ops.quantize_act(dev(x), 32), O.quantize_act(x, 32)
+    with ops.option("decode_kernel", kernel):
+        check(ops.gemv(w, a, residual=dev(res), splits=S), oracle(mode, codes, scales, act, O.VAR_GEMV, S, residual=res),
+              f"{mode} gemv")
+        if mode == "k16":
+            return
+        sp = O.segment_splits(T, M, K, None, S)
+        check(ops.gemm(w, a, torch.bfloat16, forced_splits=S),
+              oracle(mode, codes, scales, act, O.VAR_GEMM, sp, out_bf16=True), f"{mode} gemm")
+        if mode != "w8":
+            ys = ops.gemv_fanout([w, w], a)
+            ref = oracle(mode, codes, scales, act, O.VAR_FANOUT, O.gemv_splits(2 * M // 16))
+            for y in ys:
+                check(y, ref, f"{mode} fan-out")
+
+
+@pytest.mark.parametrize("T,M,K,forced", [(65, 144, 640, 1), (70, 80, 384, 4), (200, 2064, 256, 0)])
+def test_w8_general_gemm(T, M, K, forced):
+    rng = np.random.default_rng(T + M)
+    codes, scales, w = weight(rng, "w8", M, K)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    res = rng.standard_normal((T, M)).astype(np.float32)
+    a, act = ops.quantize_act(dev(x), 32), O.quantize_act(x, 32)
+    sp = O.segment_splits(T, M, K, None, forced)
+    with ops.option("gemm_kernel", 1):
+        check(ops.gemm(w, a, residual=dev(res), forced_splits=forced),
+              oracle("w8", codes, scales, act, O.VAR_GEMM, sp, residual=res), f"T={T}")

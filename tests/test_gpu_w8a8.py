@@ -115,8 +115,7 @@ def test_w8a8_gemv_long_k(T):
 
 @pytest.mark.parametrize("M,K,T", [(512, 1024, 8), (256, 2048, 16), (512, 1024, 40), (1040, 640, 300)])
 def test_w8a8_gemm(M, K, T):
-    # x_gemm_w8a8: one serial chain per output (forced split 1); T <= 16 runs
-    # on the row-wave kernel, larger T on the general GEMM
+    # x_gemm_w8a8: one serial chain per output (forced split 1)
     print(f"w8a8 gemm M={M} K={K} T={T}", flush=True)
     rng = np.random.default_rng(M * 3 + K + T)
     codes, scales, w = w8_weight(rng, M, K)
