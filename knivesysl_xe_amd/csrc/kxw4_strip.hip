@@ -217,7 +217,7 @@ __global__ __launch_bounds__(512) void strip_kernel(const StripArgs a) {
                 }
             }
         };
-        if (U == 1 || have >= U) load(std::true_type{});
+        if (have >= U) load(std::true_type{});
         else load(std::false_type{});
         wp += U * kTileBytes * TB;
         sp_ += (size_t)U * gpt * 32;
@@ -445,7 +445,7 @@ __global__ __launch_bounds__(512) void strip_kernel(const StripArgs a) {
                     if (!EDGE || i * U + UI < ntl) step(kt0 + i * U + UI, uc, edge);
                 };
                 one(std::integral_constant<int, 0>{});
-                if constexpr (U > 1) one(std::integral_constant<int, 1>{});
+                one(std::integral_constant<int, 1>{});
                 if constexpr (U > 2) {
                     one(std::integral_constant<int, 2>{});
                     one(std::integral_constant<int, 3>{});
@@ -577,7 +577,9 @@ static int st_launch(StripArgs &a, hipStream_t st) {
 // past 16 tokens, whose tiles are twice as large (T = 48: 37.0 against 46 us).
 template <int TT, int UNIT, bool BLK, int VAR, int WF>
 static int st_rw(StripArgs &a, int T, int smax, hipStream_t st) {
-    if constexpr (TT == 32) {
+    if constexpr (TT == 32 && VAR == kVarFanout) {          // (planned with 1, 8 or 16 splits)
+        return st_launch<TT, 4, 2, UNIT, BLK, VAR, WF>(a, st);
+    } else if constexpr (TT == 32) {
         return smax <= 2 ? st_launch<TT, 4, 2, UNIT, BLK, VAR, WF>(a, st) : st_launch<TT, 2, 2, UNIT, BLK, VAR, WF>(a, st);
     } else {
         if (smax == 1) {
@@ -589,7 +591,7 @@ static int st_rw(StripArgs &a, int T, int smax, hipStream_t st) {
             }
             return st_launch<TT, 4, 2, UNIT, BLK, VAR, WF>(a, st);
         }
-        if constexpr (TT == 16 && WF == kStW8) {
+        if constexpr (TT == 16 && WF == kStW8 && VAR == kVarGemm) {
             if (smax <= 4 && a.same_s && T > 16) return st_launch<TT, 2, 2, UNIT, BLK, VAR, WF>(a, st);
         }
         return st_launch<TT, 1, 2, UNIT, BLK, VAR, WF>(a, st);
@@ -629,6 +631,7 @@ static StripArgs st_take(StripArgs &a, F pick) {
 template <int UNIT, bool BLK, int VAR, int WF>
 static int st_shape(StripArgs &a, hipStream_t st) {
     constexpr int kFill = WF == kStW8 ? 2000 : 4400;
+    constexpr bool k32 = WF == kStW4 || (WF == kStW8 && VAR == kVarGemm);   // (K16 and the W8 GEMV: 16 tokens at most)
     int T = 0, smax = 1;
     a.same_s = 1;
     for (int i = 0; i < a.entries; ++i) {
@@ -636,12 +639,13 @@ static int st_shape(StripArgs &a, hipStream_t st) {
         smax = std::max(smax, a.e[i].S);
         a.same_s &= a.e[i].S == a.e[0].S;
     }
-    if (a.same_s) {
-        if (smax <= 4 && st_fills_32(a, smax, kFill)) return st_rw<32, UNIT, BLK, VAR, WF>(a, T, smax, st);
-    } else {
+    if constexpr (k32) {
+        if (a.same_s && smax <= 4 && st_fills_32(a, smax, kFill)) return st_rw<32, UNIT, BLK, VAR, WF>(a, T, smax, st);
+    }
+    if (!a.same_s) {
         // entries of one split count that fill the 32-token tiles by
         // themselves: a launch of their own
-        for (int SC = 1; SC <= 4; SC *= 2) {
+        for (int SC = 1; k32 && SC <= 4; SC *= 2) {
             if (!st_fills_32(a, SC, kFill)) continue;
             StripArgs rest = a;
             StripArgs own = st_take(rest, [&](const StripEntry &e) { return e.S == SC; });
