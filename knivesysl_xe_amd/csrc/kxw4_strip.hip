@@ -13,13 +13,17 @@
 // What bounds it. With a few tokens the weight stream (HBM), with tens of
 // them the chain (VALU: reference mode 3 operations per output and K32 unit,
 // about 1.1 ns each per SIMD, beside ~14 per unit for the zero-point fold) --
-// once neither a memory round trip nor a barrier is paid per 128-K tile. So:
+// once neither a memory round trip nor a barrier is paid per 128-K tile. So
+// (the figures of this list: four weights in turn, partly in the last-level
+// cache):
 //   * every operand of a stage (packed weights, activations, both scales)
 //     reaches LDS by direct global->LDS loads, and a stage holds U = 2 or 4
 //     tiles, double-buffered: one wait and one barrier per U tiles (one tile
 //     per stage: N = 5120, K = 17408, T = 64 per-token 57 against 42 us);
-//     deeper rings measured the same or worse, since they cost work-groups
-//     per CU (block mode N = 17408, K = 5120, T = 64: 53 against 43 us);
+//     deeper rings measured worse at tens of tokens, since they cost
+//     work-groups per CU (block mode N = 17408, K = 5120, T = 64: 53 against 43
+//     us); at a few tokens only with weights partly in the last-level cache,
+//     so whether a deeper ring helps a stream from HBM there is open;
 //   * the pointers of a stage's loads move by constants, so an issue is a
 //     handful of scalar operations (recomputed from the tile index they were
 //     ~70 per stage: 42 -> 37.6 us for the shape above);
@@ -28,14 +32,14 @@
 //     mode N = 17408, T = 64: 55 -> 48 us);
 //   * the activation scales of a lane's four tokens are read once per tile,
 //     four units at a time, in the [token][unit] order they arrive in.
-// Measured against the kernels it replaced (launches of a graph replay over
-// four weights): reference mode, N = 5120, K = 17408: T = 1 19.5 -> 14.9 us
-// (GEMV, group 64), T = 16 371 -> 22 us, T = 64 4477 -> 70 us; fan-out over
-// 34,816 rows, K = 5120, T = 1 64 -> 23.4 us; per-token N = 5120, K = 17408,
-// T = 64 118 -> 33 us (some per-token and W8 launches of up to 16 tokens stay
-// on the row-wave kernel: kxw4_route.hpp); K16 N = 5120, K = 17408: T = 1
-// 36 -> 19.2 us, T = 16 323 -> 30 us; W8 N = 17408, K = 5120: T = 8 30 -> 22
-// us, T = 64 140 -> 43 us, T = 256 401 -> 119 us.
+// Measured against the kernels it replaced (launches of a graph replay, weights
+// from HBM): reference mode, group 64, N = 5120, K = 17408: GEMV T = 1 20.9 ->
+// 17.0 us, GEMM T = 16 272 -> 24.7, T = 64 3145 -> 72.7; fan-out over 34,816
+// rows, K = 5120, T = 1 67.5 -> 25.3; per token, group 64, N = 5120, K = 17408,
+// T = 64 333 -> 36.6; K16 N = 5120, K = 17408: T = 1 36.2 -> 20.0, T = 16 325 ->
+// 32.2; W8 N = 17408, K = 5120: T = 8 30.5 -> 22.2, T = 64 140 -> 43.2, T = 256 402
+// -> 107. Launches of up to 16 tokens that another kernel runs faster stay
+// there (kxw4_route.hpp).
 #include "kxw4_device.hpp"
 #include "kxw4_internal.hpp"
 
@@ -290,8 +294,8 @@ __global__ __launch_bounds__(512) void strip_kernel(const StripArgs a) {
         if (nst > 0) issue(room);
         if (NT == 1 && RW == 1 && turn == 0) load_epilogue();           // (behind the first stage's loads)
         // (a stream of two stages has both in flight from the start; longer
-        // ones keep one ahead: two cost more than they hide, T = 1, N = 5120,
-        // K = 17408 per-token 12.3 against 10.8 us)
+        // ones keep one ahead: two took 12.3 against 10.8 us at T = 1, N = 5120,
+        // K = 17408 per token, weights partly in the last-level cache)
         const bool both = RW == 1 && nst == 2;
         if (both) issue(room - U);
         // stages whose tiles lie wholly inside the split
