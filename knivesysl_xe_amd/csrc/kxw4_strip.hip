@@ -10,12 +10,14 @@
 // stream's activation tiles, the streams are the splits of the same rows,
 // whose partials meet in LDS for the ordered sum (S = 1: one stream).
 //
-// What bounds it. With a few tokens the weight stream (HBM), with tens of
-// them the chain (VALU: reference mode 3 operations per output and K32 unit,
-// about 1.1 ns each per SIMD, beside ~14 per unit for the zero-point fold) --
-// once neither a memory round trip nor a barrier is paid per 128-K tile. So
-// (the figures of this list: four weights in turn, partly in the last-level
-// cache):
+// What bounds it. With tens of tokens in reference mode the chain (VALU: 3
+// operations per output and K32 unit, about 1.1 ns each per SIMD, beside ~14
+// per unit for the zero-point fold; 66 % busy at 27 tokens, 83 % at 512). At one
+// token, and per token where few strips leave one wave per SIMD, latency: the
+// VALU is 23-40 % busy, LDS 10 %, HBM at 2.9-3.9 TB/s, and the waves wait 38-47 %
+// of their time. Neither a memory round trip nor a barrier is paid per 128-K
+// tile (the figures of this list: four weights in turn, partly in the
+// last-level cache):
 //   * every operand of a stage (packed weights, activations, both scales)
 //     reaches LDS by direct global->LDS loads, and a stage holds U = 2 or 4
 //     tiles, double-buffered: one wait and one barrier per U tiles (one tile
